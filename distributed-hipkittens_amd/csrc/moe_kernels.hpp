@@ -10,6 +10,8 @@
 
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace hkmoe {
 
 constexpr int kRouteTok = 32;      // tokens per routing/scatter workgroup
@@ -583,26 +585,87 @@ __global__ __launch_bounds__(128) void requant_quotient_check_kernel(int* __rest
 
 // ---------------------------------------------------------------------------
 // 6. quantisers (fp32 input) used to build e4m3 operands on the device
+//
+// All are one pass over HBM (4 bytes read, 1 written per value; the per-tensor
+// one reads twice, the second time partly from the Infinity Cache), so they
+// are built to keep enough 16-byte loads in flight: every thread issues its
+// loads before it uses any.  x may be aligned to 4 bytes only and q to 1 (a
+// view into a larger tensor): the vector types below say so, and the hardware
+// takes such addresses at full width.  At 8192x7168 (5 bytes per value): groups
+// 126 -> 49 us (2.3 -> 6.0 TB/s), blocks 88 -> 50 us (5.8 TB/s), MX 54 -> 50 us
+// (5.9 TB/s), per-tensor 305 -> 95 us; what bounded them was a 512-byte wave load
+// at a time, the IEEE division per value, and 16384 same-address atomics.
 // ---------------------------------------------------------------------------
-// 1x128 groups, row-major scales [R, C/128]; one wave per group.
-__global__ __launch_bounds__(256) void quant_group_kernel(const float* __restrict__ x, int64_t rows,
-                                                          int64_t cols, uint8_t* __restrict__ q,
-                                                          float* __restrict__ s) {
-  const int lane = threadIdx.x & 63;
-  const int64_t gid = blockIdx.x * 4ll + (threadIdx.x >> 6);
-  const int64_t groups = cols / kGroup;
-  if (gid >= rows * groups) return;
-  const int64_t r = gid / groups, g = gid - r * groups;
-  const int64_t base = r * cols + g * kGroup + lane * 2;
-  const float2 v = *reinterpret_cast<const float2*>(x + base);
-  const float amax = wave_max(fmaxf(fabsf(v.x), fabsf(v.y)));
-  const float sc = scale_from_amax(amax);
-  const uint32_t qq = f32_to_e4m3(v.x / sc) | (f32_to_e4m3(v.y / sc) << 8);
-  *reinterpret_cast<uint16_t*>(q + base) = static_cast<uint16_t>(qq);
-  if (lane == 0) s[gid] = sc;
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32_u __attribute__((aligned(1)));
+
+// Maximum over the row of 16 lanes, by DPP.  fmaxf skips NaNs.
+__device__ __forceinline__ float row16_max(float v) {
+  auto step = [&](auto ctrl) __attribute__((always_inline)) {
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v),
+                                                            decltype(ctrl)::value, 0xf, 0xf, false)));
+  };
+  step(std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  step(std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  step(std::integral_constant<int, 0x141>{});  // row_half_mirror
+  step(std::integral_constant<int, 0x140>{});  // row_mirror
+  return v;
 }
 
-// 128x128 blocks of [B, R, C]; one workgroup (256 threads) per block.
+__device__ __forceinline__ float max_abs4(const f32x4& v) {
+  return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+}
+
+// Four values / sc as e4m3 bytes.  Finite values take the division-free
+// quotient (quot_e4m3 with QuotScale; over 2.7e9 random and near-midpoint fp32
+// pairs with x <= 448 sc and x / sc >= 2^-10 it never differed from x / sc) and
+// the packed conversion; a NaN or an infinite scale keeps the division and the
+// software conversion (NaN code 0x7f | sign).
+__device__ __forceinline__ uint32_t quant4(const f32x4& v, float sc, const QuotScale& qs) {
+  const bool odd = __builtin_isunordered(v.x, v.y) || __builtin_isunordered(v.z, v.w) || __builtin_isinf(sc);
+  if (__builtin_expect(odd, 0))
+    return f32_to_e4m3(v.x / sc) | (f32_to_e4m3(v.y / sc) << 8) | (f32_to_e4m3(v.z / sc) << 16) |
+           (f32_to_e4m3(v.w / sc) << 24);
+  return pack_e4m3x4(quot_e4m3(v.x, qs), quot_e4m3(v.y, qs), quot_e4m3(v.z, qs), quot_e4m3(v.w, qs));
+}
+
+// 1x128 groups, row-major scales [R, C/128].  C is a multiple of 128, so x is
+// a flat run of groups.  16 lanes per group, 8 values each (the scale's
+// reciprocal is shared by 8 values, and the maximum stays inside a DPP row),
+// two groups per lane row: four 16-byte loads in flight per thread.
+constexpr int kQuantGroups = 32;  // groups per workgroup
+__global__ __launch_bounds__(256) void quant_group_kernel(const float* __restrict__ x, int64_t groups,
+                                                          uint8_t* __restrict__ q, float* __restrict__ s) {
+  const int l = threadIdx.x & 15;
+  const int64_t g0 = blockIdx.x * static_cast<int64_t>(kQuantGroups) + (threadIdx.x >> 4);
+  f32x4 v[2][2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int64_t g = g0 + 16 * u;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      v[u][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (g < groups)
+        v[u][h] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(x + g * kGroup + 64 * h + 4 * l));
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int64_t g = g0 + 16 * u;
+    const float sc = scale_from_amax(row16_max(fmaxf(max_abs4(v[u][0]), max_abs4(v[u][1]))));
+    const QuotScale qs = quot_scale(sc);
+    if (g < groups) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<u32_u*>(q + g * kGroup + 64 * h + 4 * l) = quant4(v[u][h], sc, qs);
+      if (l == 0) s[g] = sc;
+    }
+  }
+}
+
+// 128x128 blocks of [B, R, C]; one workgroup (256 threads) per block, the
+// block held in registers (64 per thread) between the maximum and the
+// conversion, so x is read once.
 __global__ __launch_bounds__(256) void quant_block_kernel(const float* __restrict__ x, int64_t rows,
                                                           int64_t cols, uint8_t* __restrict__ q,
                                                           float* __restrict__ s) {
@@ -616,33 +679,81 @@ __global__ __launch_bounds__(256) void quant_block_kernel(const float* __restric
   uint8_t* qb = q + (b * rows + bi * kGroup) * cols + bj * kGroup;
   // thread: rows (tid/32) + 8*u, columns 4*(tid%32) .. +3
   const int cr = threadIdx.x >> 5, cc = (threadIdx.x & 31) * 4;
+  f32x4 v[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u)
+    v[u] = __builtin_nontemporal_load(
+        reinterpret_cast<const f32x4_u*>(xb + static_cast<int64_t>(cr + 8 * u) * cols + cc));
   float m = 0.0f;
-  for (int u = 0; u < 16; ++u) {
-    const float4 v = *reinterpret_cast<const float4*>(xb + static_cast<int64_t>(cr + 8 * u) * cols + cc);
-    m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-  }
+#pragma unroll
+  for (int u = 0; u < 16; ++u) m = fmaxf(m, max_abs4(v[u]));
   m = wave_max(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  const float amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const float sc = scale_from_amax(amax);
-  for (int u = 0; u < 16; ++u) {
-    const int64_t off = static_cast<int64_t>(cr + 8 * u) * cols + cc;
-    const float4 v = *reinterpret_cast<const float4*>(xb + off);
-    const uint32_t qq = f32_to_e4m3(v.x / sc) | (f32_to_e4m3(v.y / sc) << 8) |
-                        (f32_to_e4m3(v.z / sc) << 16) | (f32_to_e4m3(v.w / sc) << 24);
-    *reinterpret_cast<uint32_t*>(qb + off) = qq;
-  }
+  const float sc = scale_from_amax(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+  const QuotScale qs = quot_scale(sc);
+#pragma unroll
+  for (int u = 0; u < 16; ++u)
+    *reinterpret_cast<u32_u*>(qb + static_cast<int64_t>(cr + 8 * u) * cols + cc) = quant4(v[u], sc, qs);
   if (threadIdx.x == 0) s[blk] = sc;
 }
 
-__global__ __launch_bounds__(256) void amax_kernel(const float* __restrict__ x, int64_t n,
-                                                   float* amax) {
+// Per-tensor: the maximum over all values, then the conversion.
+constexpr int kAmaxUnroll = 4;  // 16-byte loads in flight per thread
+
+// max |x| over n values, seen by a workgroup of THREADS threads that reads the
+// 4-value chunks first, first + step, ...; the last n % 4 values go to the
+// first chunk's owner.
+template <int THREADS>
+__device__ __forceinline__ float amax_range(const float* __restrict__ x, int64_t n, int64_t first, int64_t step) {
+  const int64_t n4 = n / 4;
   float m = 0.0f;
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * 256)
-    m = fmaxf(m, fabsf(x[i]));
+  int64_t i = first;
+  for (; i + (kAmaxUnroll - 1) * step < n4; i += kAmaxUnroll * step) {
+    f32x4 v[kAmaxUnroll];
+#pragma unroll
+    for (int u = 0; u < kAmaxUnroll; ++u) v[u] = reinterpret_cast<const f32x4_u*>(x)[i + u * step];
+#pragma unroll
+    for (int u = 0; u < kAmaxUnroll; ++u) m = fmaxf(m, max_abs4(v[u]));
+  }
+  for (; i < n4; i += step) m = fmaxf(m, max_abs4(reinterpret_cast<const f32x4_u*>(x)[i]));
+  if (first == 0)
+    for (int64_t j = 4 * n4; j < n; ++j) m = fmaxf(m, fabsf(x[j]));
+  __shared__ float red[THREADS / 64];
   m = wave_max(m);
-  if ((threadIdx.x & 63) == 0) atomicMax(reinterpret_cast<unsigned int*>(amax), __float_as_uint(m));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < THREADS / 64; ++w) m = fmaxf(m, red[w]);
+  return m;
+}
+
+// Chunks first, first + step, ... of x converted with scale sc.
+__device__ __forceinline__ void quant_range(const float* __restrict__ x, int64_t n, int64_t first, int64_t step,
+                                            float sc, uint8_t* __restrict__ q) {
+  const QuotScale qs = quot_scale(sc);
+  const int64_t n4 = n / 4;
+  int64_t i = first;
+  for (; i + (kAmaxUnroll - 1) * step < n4; i += kAmaxUnroll * step) {
+    f32x4 v[kAmaxUnroll];
+#pragma unroll
+    for (int u = 0; u < kAmaxUnroll; ++u) v[u] = reinterpret_cast<const f32x4_u*>(x)[i + u * step];
+#pragma unroll
+    for (int u = 0; u < kAmaxUnroll; ++u) *reinterpret_cast<u32_u*>(q + 4 * (i + u * step)) = quant4(v[u], sc, qs);
+  }
+  for (; i < n4; i += step)
+    *reinterpret_cast<u32_u*>(q + 4 * i) = quant4(reinterpret_cast<const f32x4_u*>(x)[i], sc, qs);
+  if (first == 0)
+    for (int64_t j = 4 * n4; j < n; ++j) q[j] = static_cast<uint8_t>(f32_to_e4m3(x[j] / sc));
+}
+
+// One atomic per workgroup at most: a workgroup whose maximum is not above the
+// one already published skips it (the value only grows, so a stale read costs
+// an atomic, not the result).
+__global__ __launch_bounds__(256) void amax_kernel(const float* __restrict__ x, int64_t n, float* amax) {
+  const float m = amax_range<256>(x, n, blockIdx.x * 256ll + threadIdx.x, static_cast<int64_t>(gridDim.x) * 256);
+  if (threadIdx.x == 0 && m > __hip_atomic_load(amax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(reinterpret_cast<unsigned int*>(amax), __float_as_uint(m));
 }
 
 __global__ void fill_f32_kernel(float* p, float v) { *p = v; }
@@ -653,8 +764,17 @@ __global__ __launch_bounds__(256) void quant_tensor_kernel(const float* __restri
                                                            float* __restrict__ s) {
   const float sc = scale_from_amax(*amax);
   if (blockIdx.x == 0 && threadIdx.x == 0) s[0] = sc;
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * 256)
-    q[i] = static_cast<uint8_t>(f32_to_e4m3(x[i] / sc));
+  quant_range(x, n, blockIdx.x * 256ll + threadIdx.x, static_cast<int64_t>(gridDim.x) * 256, sc, q);
+}
+
+// Small tensors: one launch.  Every workgroup takes the maximum over the whole
+// tensor (its XCD's L2 holds it) and converts its own share.
+constexpr int64_t kQuantSmall = 1 << 17;  // values
+__global__ __launch_bounds__(1024) void quant_tensor_small_kernel(const float* __restrict__ x, int64_t n,
+                                                                  uint8_t* __restrict__ q, float* __restrict__ s) {
+  const float sc = scale_from_amax(amax_range<1024>(x, n, threadIdx.x, 1024));
+  if (blockIdx.x == 0 && threadIdx.x == 0) s[0] = sc;
+  quant_range(x, n, blockIdx.x * 1024ll + threadIdx.x, static_cast<int64_t>(gridDim.x) * 1024, sc, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -666,23 +786,35 @@ __global__ __launch_bounds__(256) void quant_tensor_kernel(const float* __restri
 // -- and q = e4m3(x * 2^(127 - s)), an exact power-of-two scaling followed by
 // one RNE conversion (|x * 2^(127-s)| < 2, so the saturating clamp never acts).
 // Reference behaviour: 4_wave.cu:296-321, 368-373.
+// Each workgroup owns 1024 quads; a thread's four loads are in flight together.
+constexpr int kMxQuads = 1024;
 __global__ __launch_bounds__(256) void quant_mx_kernel(const float* __restrict__ x, int64_t blocks,
                                                        uint8_t* __restrict__ q, uint8_t* __restrict__ s) {
   const int64_t quads = blocks * 8;
-  // quad i = lane i % 8 of block i / 8; the 8 lanes of a block sit in one wave
-  // (i % 8 == threadIdx.x % 8) and pass the loop test together
-  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < quads; i += static_cast<int64_t>(gridDim.x) * 256) {
-    const float4 v = *reinterpret_cast<const float4*>(x + 4 * i);
-    float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+  // quad i = lane i % 8 of block i / 8; the 8 lanes of a block sit in one DPP
+  // row (i % 8 == threadIdx.x % 8) and are in or out of range together
+  const int64_t i0 = blockIdx.x * static_cast<int64_t>(kMxQuads) + threadIdx.x;
+  f32x4 v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (i0 + 256 * u < quads) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(x) + i0 + 256 * u);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t i = i0 + 256 * u;
+    float m = max_abs4(v[u]);
     m = fmaxf(m, __shfl_xor(m, 1, kWave));
     m = fmaxf(m, __shfl_xor(m, 2, kWave));
     m = fmaxf(m, __shfl_xor(m, 4, kWave));
     const uint32_t e = min((__float_as_uint(m) >> 23) & 0xffu, 254u);
     const int sh = 127 - static_cast<int>(e);
-    *reinterpret_cast<uint32_t*>(q + 4 * i) =
-        pack_e4m3x4(__builtin_amdgcn_ldexpf(v.x, sh), __builtin_amdgcn_ldexpf(v.y, sh),
-                    __builtin_amdgcn_ldexpf(v.z, sh), __builtin_amdgcn_ldexpf(v.w, sh));
-    if ((i & 7) == 0) s[i >> 3] = static_cast<uint8_t>(e);
+    if (i < quads) {
+      *reinterpret_cast<u32_u*>(q + 4 * i) =
+          pack_e4m3x4(__builtin_amdgcn_ldexpf(v[u].x, sh), __builtin_amdgcn_ldexpf(v[u].y, sh),
+                      __builtin_amdgcn_ldexpf(v[u].z, sh), __builtin_amdgcn_ldexpf(v[u].w, sh));
+      if ((i & 7) == 0) s[i >> 3] = static_cast<uint8_t>(e);
+    }
   }
 }
 
