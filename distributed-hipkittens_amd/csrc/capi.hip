@@ -17,6 +17,7 @@
 #include "../../include/hkmoe.h"
 #include "gemm_fp8.hpp"
 #include "gemm_narrow.hpp"
+#include "gemm_skinny.hpp"
 #include "gemm_small.hpp"
 #include "moe_kernels.hpp"
 
@@ -145,6 +146,11 @@ int device_cus() {
   return cus[dev];
 }
 
+int env_int(const char* name, int dflt) {
+  const char* v = std::getenv(name);
+  return (v && *v) ? std::atoi(v) : dflt;
+}
+
 size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 int route_blocks(int64_t t) { return static_cast<int>((t + kRouteTok - 1) / kRouteTok); }
@@ -175,21 +181,190 @@ std::atomic<int> g_dense_mfma{32};
 
 // The dense GEMM on 128x128 tiles (gemm_small.hpp): one workgroup per tile,
 // the grid a whole number of 4x8 tile blocks.
-template <bool F32OUT, bool M32>
+template <bool F32OUT, bool M32, bool MX>
 int launch_gemm_small(const SmallGemmParams& p, hipStream_t stream) {
   static bool attr_set[kMaxDevices] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_fp8_small<F32OUT, M32>;
+  auto kern = gemm_fp8_small<F32OUT, M32, MX>;
+  constexpr int lds = sm_lds_bytes(MX);
   if (dev >= 0 && dev < kMaxDevices && !attr_set[dev]) {
     const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, kSmLdsBytes);
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (err != hipSuccess) return fail(HKMOE_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(err));
     attr_set[dev] = true;
   }
   const int grid = ((p.m_tiles + 3) / 4) * p.nbn * 32;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(kSmThreads), kSmLdsBytes, stream, p);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(kSmThreads), lds, stream, p);
   return check_launch("gemm_fp8_small");
+}
+
+template <int MF, int NF, int NW, bool MX, bool F32OUT>
+int launch_gemm_skinny(const SkinnyParams& p, hipStream_t stream) {
+  static bool attr_set[kMaxDevices] = {false};
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  auto kern = gemm_fp8_skinny<MF, NF, NW, MX, F32OUT>;
+  constexpr int lds = sk_lds_bytes(MF, NF, NW, MX);
+  if (dev >= 0 && dev < kMaxDevices && !attr_set[dev]) {
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (err != hipSuccess) return fail(HKMOE_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(err));
+    attr_set[dev] = true;
+  }
+  const int64_t grid = static_cast<int64_t>(p.strips) * p.m_blocks;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(NW * 64), lds, stream, p);
+  return check_launch("gemm_fp8_skinny");
+}
+template <int MF, int NF, int NW, bool MX>
+int launch_gemm_skinny(SkinnyParams p, bool f32out, hipStream_t stream) {
+  p.strips = p.n / (16 * NF);
+  p.m_blocks = (p.m + 16 * MF - 1) / (16 * MF);
+  return f32out ? launch_gemm_skinny<MF, NF, NW, MX, true>(p, stream) : launch_gemm_skinny<MF, NF, NW, MX, false>(p, stream);
+}
+
+// Estimated times (us) of the dense kernels, from which the dense GEMM picks one:
+// rounds of workgroups over the CUs x (ramp + K steps x time per step), or B's
+// stream from HBM where that is longer (a tenth of the compute term breaks ties
+// there).  The constants are fits to graph-replayed launches with three operand
+// copies; on 256 other shapes (M = 1 .. 10000, N = 512 .. 7168, K = 512 .. 14336,
+// both outputs and modes) the pick costs 0.4% over the best kernel on average,
+// 21% at worst.
+//   split-K strips against 128x128 tiles: 17x8192x2048 5.2 / 11.0 us, 64x2048x8192
+//     7.5 / 33, 256x4096x4096 11.6 / 19, 1024x1024x4096 11.6 / 19 (and losing:
+//     1024x4096x4096 40 / 22)
+//   128x128 against 256x256 tiles: 2048^3 14.5 / 25.6 us, 2048x4096x4096 43 / 48,
+//     4096^3 84 / 52, 2048x7168x2048 46 / 30
+// MX: the scaled MFMA's steps take longer in every kernel, most in the 128x128 one.
+enum class DenseKernel { kStrip11, kStrip21, kStrip12, kStrip22, kStrip24, kStrip44, kTile128, kTile256 };
+
+// Tile blocks of the dense 256x256 kernel: 2^b M tiles x 32 / 2^b N tiles, one
+// block per XCD and round.  4 x 8 unless another shape needs fewer rounds: a
+// block wider than N (or taller than M) leaves workgroups idle (12878x1024x1664,
+// 51 x 4 tiles, fp32 out: 48.5 us in 4 x 8 blocks, whose right half is empty,
+// 30.8 in 8 x 4).
+int dense_block_log2(int64_t m, int64_t n, int64_t* rounds) {
+  const uint64_t mt = (m + kBM - 1) / kBM, nt = n / kBN;
+  int best = 2;
+  uint64_t best_r = UINT64_MAX;
+  for (int b : {2, 3, 1, 4, 5, 0}) {
+    const uint64_t blocks = ((mt + (1u << b) - 1) >> b) * ((nt + (32u >> b) - 1) >> (5 - b));
+    if ((blocks + 7) / 8 < best_r) best = b, best_r = (blocks + 7) / 8;
+  }
+  *rounds = static_cast<int64_t>(best_r);
+  return best;
+}
+
+DenseKernel pick_dense(int64_t m, int64_t n, int64_t k, bool f32out, bool mx) {
+  const double ks = static_cast<double>(k / kBK), cus = device_cus(), nk = static_cast<double>(n) * k;
+  const uint64_t um = m, un = n, ncu = device_cus();
+  DenseKernel best = DenseKernel::kTile256;
+  double best_t = 0;
+  auto offer = [&](DenseKernel kern, double compute, double hbm) {
+    const double t = std::max(compute, hbm) + 0.1 * compute;
+    if (kern == DenseKernel::kTile256 || t < best_t) best = kern, best_t = t;
+  };
+  {
+    const double tiles = static_cast<double>((m + kBM - 1) / kBM) * (n / kBN);
+    const double step = tiles <= cus / 4 ? (mx ? 1.12 : 0.95) : tiles <= cus / 2 ? (mx ? 1.27 : 1.13) : (mx ? 1.45 : 1.3);
+    int64_t rounds;
+    (void)dense_block_log2(m, n, &rounds);
+    offer(DenseKernel::kTile256, 5.4 + static_cast<double>(rounds) * ((f32out ? 11 : 5) + ks * step), 0);
+  }
+  {
+    const uint64_t tiles = ((um + kSmTile - 1) / kSmTile) * (un / kSmTile);
+    const double full = static_cast<double>(tiles / ncu), part = static_cast<double>(tiles % ncu);
+    const double busy = mx ? 0.74 : 0.58, idle = mx ? 0.68 : 0.47;  // per step, chip full / half full
+    const double ramp = f32out ? 4.8 : 2.3;
+    offer(DenseKernel::kTile128,
+          2 + full * (ramp + ks * busy) + (part > 0 ? ramp + ks * (part <= cus / 2 ? idle : busy) : 0), 3 + nk / 2.0e6);
+  }
+  const struct {
+    DenseKernel kern;
+    int rows_log2, cols_log2, waves_log2;
+    double ramp, step;
+  } strips[] = {{DenseKernel::kStrip11, 4, 4, 3, 1.6, 0.055}, {DenseKernel::kStrip21, 5, 4, 3, 1.7, 0.075},
+                {DenseKernel::kStrip12, 4, 5, 3, 1.7, 0.075}, {DenseKernel::kStrip22, 5, 5, 3, 1.85, 0.085},
+                {DenseKernel::kStrip24, 5, 6, 2, 2.4, 0.13},  {DenseKernel::kStrip44, 6, 6, 2, 3.1, 0.215}};
+  for (const auto& c : strips) {
+    const uint64_t wgs = ((um + (1u << c.rows_log2) - 1) >> c.rows_log2) * (un >> c.cols_log2);
+    const double rounds = static_cast<double>((wgs + ncu - 1) / ncu);
+    const double steps = static_cast<double>(((k / kBK + (1 << c.waves_log2) - 1) >> c.waves_log2) << c.waves_log2);
+    offer(c.kern, (mx ? 1.6 : 1.3) + rounds * (c.ramp + steps * c.step * (mx ? 1.1 : 1.0)), 3 + nk / 5.5e6);
+  }
+  return best;
+}
+
+// The dense GEMM (a, b, c and shapes checked by the caller).  MX: scale_a and
+// scale_b are the packed exponent words.
+template <bool MX>
+int launch_dense(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, const float* scale_a,
+                 const float* scale_b, int out_dtype, hipStream_t s) {
+  const bool f32out = out_dtype == HKMOE_F32;
+  const int32_t m64 = static_cast<int32_t>((m + 63) / 64 * 64);
+  const DenseKernel kern = pick_dense(m, n, k, f32out, MX);
+  if (kern < DenseKernel::kTile128) {
+    SkinnyParams q{};
+    q.a = static_cast<const uint8_t*>(a);
+    q.b = static_cast<const uint8_t*>(b);
+    q.c = c;
+    q.a_scale = scale_a;
+    q.b_scale = scale_b;
+    q.m = static_cast<int32_t>(m);
+    q.n = static_cast<int32_t>(n);
+    q.k = static_cast<int32_t>(k);
+    q.m64 = m64;
+    switch (kern) {
+      case DenseKernel::kStrip11: return launch_gemm_skinny<1, 1, 8, MX>(q, f32out, s);
+      case DenseKernel::kStrip21: return launch_gemm_skinny<2, 1, 8, MX>(q, f32out, s);
+      case DenseKernel::kStrip12: return launch_gemm_skinny<1, 2, 8, MX>(q, f32out, s);
+      case DenseKernel::kStrip22: return launch_gemm_skinny<2, 2, 8, MX>(q, f32out, s);
+      case DenseKernel::kStrip24: return launch_gemm_skinny<2, 4, 4, MX>(q, f32out, s);
+      default: return launch_gemm_skinny<4, 4, 4, MX>(q, f32out, s);
+    }
+  }
+  if (kern == DenseKernel::kTile128) {
+    SmallGemmParams q{};
+    q.a = static_cast<const uint8_t*>(a);
+    q.b = static_cast<const uint8_t*>(b);
+    q.c = c;
+    q.a_scale = scale_a;
+    q.b_scale = scale_b;
+    q.m = static_cast<int32_t>(m);
+    q.n = static_cast<int32_t>(n);
+    q.k = static_cast<int32_t>(k);
+    q.m64 = m64;
+    q.a_bytes = static_cast<uint32_t>(std::min<int64_t>(m * k, 0xffffffffll));
+    q.b_bytes = static_cast<uint32_t>(std::min<int64_t>(n * k, 0xffffffffll));
+    q.m_tiles = static_cast<int32_t>((m + kSmTile - 1) / kSmTile);
+    q.n_tiles = static_cast<int32_t>(n / kSmTile);
+    q.nbn = (q.n_tiles + 7) / 8;
+    if constexpr (MX) {
+      return f32out ? launch_gemm_small<true, false, true>(q, s) : launch_gemm_small<false, false, true>(q, s);
+    } else {
+      if (g_dense_mfma.load() == 32)
+        return f32out ? launch_gemm_small<true, true, false>(q, s) : launch_gemm_small<false, true, false>(q, s);
+      return f32out ? launch_gemm_small<true, false, false>(q, s) : launch_gemm_small<false, false, false>(q, s);
+    }
+  }
+  GemmParams p{};
+  p.a = static_cast<const uint8_t*>(a);
+  p.b = static_cast<const uint8_t*>(b);
+  p.c = c;
+  p.a_scale = scale_a;
+  p.b_scale = scale_b;
+  p.rows = m;
+  p.a_rows = m;
+  p.as_rs = m64;  // MX words per K step
+  p.num_experts = 1;
+  p.K = static_cast<int32_t>(k);
+  p.nb = static_cast<int32_t>(n);
+  p.n_out = static_cast<int32_t>(n);
+  p.n_tiles = static_cast<int32_t>(n / kBN);
+  int64_t rounds;
+  p.blk_m_log2 = dense_block_log2(m, n, &rounds);
+  constexpr Scale kSc = MX ? Scale::kMX : Scale::kTensor;
+  return f32out ? launch_gemm<Epi::kStoreF32, kSc>(p, s) : launch_gemm<Epi::kStoreBf16, kSc>(p, s);
 }
 
 // Prefetch depth of the narrow kernel for K / 128 steps: the largest of 8, 4,
@@ -239,10 +414,6 @@ int launch_narrow(GemmParams p, hipStream_t stream, int grid) {
 struct NarrowConfig {
   int cus, max_rows, share;
 };
-int env_int(const char* name, int dflt) {
-  const char* v = std::getenv(name);
-  return (v && *v) ? std::atoi(v) : dflt;
-}
 std::mutex g_narrow_mu;
 NarrowConfig& narrow_config_ref() {
   static NarrowConfig cfg = [] {
@@ -437,43 +608,7 @@ int hkmoe_gemm_fp8(const void* a, const void* b, void* c, int64_t m, int64_t n, 
              "gemm_fp8: operand too large for 32-bit buffer offsets (M*K and N*K must be < 2^32)");
   HK_REQUIRE(out_dtype == HKMOE_BF16 || out_dtype == HKMOE_F32, "gemm_fp8: bad out_dtype %d", out_dtype);
   if (m == 0) return HKMOE_OK;
-  auto s = static_cast<hipStream_t>(stream);
-  // Fewer 256x256 tiles than two per CU: 128x128 tiles, one workgroup each.
-  if (((m + kBM - 1) / kBM) * (n / kBN) < 2ll * device_cus()) {
-    SmallGemmParams q{};
-    q.a = static_cast<const uint8_t*>(a);
-    q.b = static_cast<const uint8_t*>(b);
-    q.c = c;
-    q.a_scale = scale_a;
-    q.b_scale = scale_b;
-    q.m = static_cast<int32_t>(m);
-    q.n = static_cast<int32_t>(n);
-    q.k = static_cast<int32_t>(k);
-    q.a_bytes = static_cast<uint32_t>(std::min<int64_t>(m * k, 0xffffffffll));
-    q.b_bytes = static_cast<uint32_t>(std::min<int64_t>(n * k, 0xffffffffll));
-    q.m_tiles = static_cast<int32_t>((m + kSmTile - 1) / kSmTile);
-    q.n_tiles = static_cast<int32_t>(n / kSmTile);
-    q.nbn = (q.n_tiles + 7) / 8;
-    if (g_dense_mfma.load() == 32)
-      return out_dtype == HKMOE_BF16 ? launch_gemm_small<false, true>(q, s) : launch_gemm_small<true, true>(q, s);
-    return out_dtype == HKMOE_BF16 ? launch_gemm_small<false, false>(q, s) : launch_gemm_small<true, false>(q, s);
-  }
-  GemmParams p{};
-  p.a = static_cast<const uint8_t*>(a);
-  p.b = static_cast<const uint8_t*>(b);
-  p.c = c;
-  p.a_scale = scale_a;
-  p.b_scale = scale_b;
-  p.rows = m;
-  p.a_rows = m;
-  p.num_experts = 1;
-  p.K = static_cast<int32_t>(k);
-  p.nb = static_cast<int32_t>(n);
-  p.n_out = static_cast<int32_t>(n);
-  p.n_tiles = static_cast<int32_t>(n / kBN);
-  p.blk_m_log2 = 2;  // 4 x 8 tile blocks
-  return out_dtype == HKMOE_BF16 ? launch_gemm<Epi::kStoreBf16, Scale::kTensor>(p, s)
-                                 : launch_gemm<Epi::kStoreF32, Scale::kTensor>(p, s);
+  return launch_dense<false>(a, b, c, m, n, k, scale_a, scale_b, out_dtype, static_cast<hipStream_t>(stream));
 }
 
 int hkmoe_route_blocks(int64_t num_tokens) { return route_blocks(num_tokens); }
@@ -1201,26 +1336,9 @@ int hkmoe_gemm_mx(const void* a, const void* a_scale, const void* b, const void*
              "gemm_mx: operand too large for 32-bit buffer offsets (M*K and N*K must be < 2^32)");
   HK_REQUIRE(out_dtype == HKMOE_BF16 || out_dtype == HKMOE_F32, "gemm_mx: bad out_dtype %d", out_dtype);
   if (m == 0) return HKMOE_OK;
-  GemmParams p{};
-  p.a = static_cast<const uint8_t*>(a);
-  p.b = static_cast<const uint8_t*>(b);
-  p.c = c;
-  p.a_scale = static_cast<const float*>(a_scale);
-  p.b_scale = static_cast<const float*>(b_scale);
-  p.rows = m;
-  p.a_rows = m;
-  p.as_rs = m64;
-  p.num_experts = 1;
-  p.K = static_cast<int32_t>(k);
-  p.nb = static_cast<int32_t>(n);
-  p.n_out = static_cast<int32_t>(n);
-  p.n_tiles = static_cast<int32_t>(n / kBN);
-  p.blk_m_log2 = 2;  // 4 x 8 tile blocks
-  auto st = static_cast<hipStream_t>(stream);
-  return out_dtype == HKMOE_BF16 ? launch_gemm<Epi::kStoreBf16, Scale::kMX>(p, st)
-                                 : launch_gemm<Epi::kStoreF32, Scale::kMX>(p, st);
+  return launch_dense<true>(a, b, c, m, n, k, static_cast<const float*>(a_scale),
+                            static_cast<const float*>(b_scale), out_dtype, static_cast<hipStream_t>(stream));
 }
-
 
 int64_t hkmoe_mx_words_per_step(int64_t rows, int32_t num_experts) {
   return rows < 0 || num_experts < 1 ? 0 : mx_words_per_step(rows, num_experts);

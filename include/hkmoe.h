@@ -71,8 +71,8 @@ int hkmoe_gemm_fp8(const void* a, const void* b, void* c, int64_t m, int64_t n, 
                    hkmoe_stream_t stream);
 
 /*
- * MFMA shape of hkmoe_gemm_fp8's kernel for small problems (fewer 256x256 tiles
- * than two per CU, e.g. 2048^3), which runs 128x128 tiles: 16 for
+ * MFMA shape of hkmoe_gemm_fp8's kernel for mid-sized problems (too few 256x256
+ * tiles to fill the chip, e.g. 2048^3), which runs 128x128 tiles: 16 for
  * v_mfma_f32_16x16x128_f8f6f4, 32 for v_mfma_f32_32x32x64_f8f6f4 (the default:
  * 4-7% faster at 2048^3 and similar shapes).
  * Both give the same sums (fp32 accumulation in another order).  Replaces the
