@@ -14,8 +14,15 @@ GROUP = 128
 
 def _check_dev(*ts):
     for t in ts:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError("hkmoe: tensors must live on a GPU device")
+
+
+# Outputs are allocated from an input (empty_like / new_empty): a third of the
+# host time of torch.empty with a shape, a dtype and a device to convert, which is what a
+# small call waits for.
+def _like(x, dtype):
+    return torch.empty_like(x, dtype=dtype, memory_format=torch.contiguous_format)
 
 
 # ----------------------------------------------------------------------------
@@ -25,8 +32,8 @@ def quant_group(x):
     """fp32 [R, C] -> (e4m3 [R, C], fp32 scales [R, C/128]), 1x128 groups."""
     _check_dev(x)
     x = x.float().contiguous()
-    q = torch.empty(x.shape, dtype=F8, device=x.device)
-    s = torch.empty((x.shape[0], x.shape[1] // GROUP), dtype=torch.float32, device=x.device)
+    q = _like(x, F8)
+    s = x.new_empty((x.shape[0], x.shape[1] // GROUP))
     tk_kernel.dispatch_quant_group(x, q, s)
     return q, s
 
@@ -35,9 +42,8 @@ def quant_block(w):
     """fp32 [..., R, C] -> (e4m3, fp32 scales [..., R/128, C/128]), 128x128 blocks."""
     _check_dev(w)
     w = w.float().contiguous()
-    q = torch.empty(w.shape, dtype=F8, device=w.device)
-    s = torch.empty((*w.shape[:-2], w.shape[-2] // GROUP, w.shape[-1] // GROUP),
-                    dtype=torch.float32, device=w.device)
+    q = _like(w, F8)
+    s = w.new_empty((*w.shape[:-2], w.shape[-2] // GROUP, w.shape[-1] // GROUP))
     tk_kernel.dispatch_quant_block(w.reshape(-1, w.shape[-2], w.shape[-1]), q, s)
     return q, s
 
@@ -46,9 +52,9 @@ def quant_tensor(x):
     """fp32 tensor -> (e4m3, fp32 scale [1]), s = amax/448."""
     _check_dev(x)
     x = x.float().contiguous()
-    q = torch.empty(x.shape, dtype=F8, device=x.device)
-    s = torch.empty(1, dtype=torch.float32, device=x.device)
-    ws = torch.empty(1, dtype=torch.float32, device=x.device)
+    q = _like(x, F8)
+    s = x.new_empty((1,))
+    ws = x.new_empty((1,))
     tk_kernel.dispatch_quant_tensor(x, q, s, ws)
     return q, s
 
@@ -56,7 +62,7 @@ def quant_tensor(x):
 def gemm_fp8(a_q, b_q, scale_a=None, scale_b=None, out_dtype=torch.bfloat16):
     """C = (sa*sb) A . B^T for e4m3 A [M,K], B [N,K]."""
     _check_dev(a_q, b_q)
-    c = torch.empty((a_q.shape[0], b_q.shape[0]), dtype=out_dtype, device=a_q.device)
+    c = a_q.new_empty((a_q.shape[0], b_q.shape[0]), dtype=out_dtype)
     tk_kernel.dispatch_gemm_fp8(a_q, b_q, c, scale_a, scale_b)
     return c
 
@@ -68,8 +74,8 @@ def quant_mx(x):
     """fp32 [R, C] -> (e4m3 [R, C], e8m0 exponents uint8 [R, C/32])."""
     _check_dev(x)
     x = x.float().contiguous()
-    q = torch.empty(x.shape, dtype=F8, device=x.device)
-    s = torch.empty((x.shape[0], x.shape[1] // 32), dtype=torch.uint8, device=x.device)
+    q = _like(x, F8)
+    s = x.new_empty((x.shape[0], x.shape[1] // 32), dtype=torch.uint8)
     tk_kernel.dispatch_quant_mx(x, q, s)
     return q, s
 
@@ -79,7 +85,7 @@ def mx_pack_scales(s):
     _check_dev(s)
     s = s.contiguous()
     rows, cols = s.shape[0], s.shape[1] * 32
-    packed = torch.empty((cols // 128, (rows + 63) // 64 * 64), dtype=torch.int32, device=s.device)
+    packed = s.new_empty((cols // 128, (rows + 63) // 64 * 64), dtype=torch.int32)
     tk_kernel.dispatch_mx_pack_scales(s, cols, packed)
     return packed
 
@@ -87,7 +93,7 @@ def mx_pack_scales(s):
 def gemm_mx(a_q, a_packed, b_q, b_packed, out_dtype=torch.float32):
     """C = A . B^T with 1x32 e8m0 block scales (packed by mx_pack_scales)."""
     _check_dev(a_q, b_q)
-    c = torch.empty((a_q.shape[0], b_q.shape[0]), dtype=out_dtype, device=a_q.device)
+    c = a_q.new_empty((a_q.shape[0], b_q.shape[0]), dtype=out_dtype)
     tk_kernel.dispatch_gemm_mx(a_q, a_packed, b_q, b_packed, c)
     return c
 
@@ -117,7 +123,7 @@ def moe_forward(x_q, x_scale, logits, w13_q, w13_scale, w2_q, w2_scale, top_k,
     e, two_i, _ = w13_q.shape
     mode = tk_kernel.SCALE_TENSOR if x_scale.numel() == 1 and x_scale.dim() <= 1 else tk_kernel.SCALE_BLOCK
     if out is None:
-        out = torch.empty((t, hidden), dtype=torch.bfloat16, device=x_q.device)
+        out = x_q.new_empty((t, hidden), dtype=torch.bfloat16)
     need = tk_kernel.moe_workspace_size(t, e, top_k, hidden, two_i // 2, mode)
     if workspace is None or workspace.numel() < need:
         workspace = torch.empty(need, dtype=torch.uint8, device=x_q.device)
@@ -369,7 +375,7 @@ class MoELayerMX:
     def __call__(self, x_q, x_e8m0, logits, out=None):
         t = x_q.shape[0]
         if out is None:
-            out = torch.empty((t, self.hidden), dtype=torch.bfloat16, device=x_q.device)
+            out = x_q.new_empty((t, self.hidden), dtype=torch.bfloat16)
         tk_kernel.dispatch_moe_mx(x_q, x_e8m0, logits, self.w13_q, self.w13_words, self.w2_q, self.w2_words,
                                   self.top_k, out, self.workspace(t, x_q.device), packed=self.packed)
         return out
