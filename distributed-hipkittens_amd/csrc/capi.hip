@@ -367,40 +367,64 @@ int launch_dense(const void* a, const void* b, void* c, int64_t m, int64_t n, in
   return f32out ? launch_gemm<Epi::kStoreF32, kSc>(p, s) : launch_gemm<Epi::kStoreBf16, kSc>(p, s);
 }
 
-// Prefetch depth of the narrow kernel for K / 128 steps: the largest of 8, 4,
-// 2 that divides the step count (0: the narrow path cannot run this K: an odd
-// step count, or more than 64 steps).
-int narrow_depth(int k_steps) {
-  if (k_steps > kNarrowMaxSteps) return 0;  // an item's scales must fit one LDS buffer
-  return k_steps % 8 == 0 ? 8 : k_steps % 4 == 0 ? 4 : k_steps % 2 == 0 ? 2 : 0;
-}
-
-template <Epi EPI, int P>
-int launch_narrow_p(const GemmParams& p, hipStream_t stream, int grid) {
+template <Epi EPI, Scale SC, int P, int NW, int ROWS, bool PAD>
+int launch_narrow_v(const GemmParams& p, hipStream_t stream, int grid) {
   static bool attr_set[kMaxDevices] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
-  auto kern = gemm_fp8_narrow<EPI, P>;
-  constexpr int lds = narrow_lds_bytes(P);
+  auto kern = gemm_fp8_narrow<EPI, SC, P, NW, ROWS, PAD>;
+  using G = NarrowGeo<SC, P, NW, ROWS>;
   if (dev >= 0 && dev < kMaxDevices && !attr_set[dev]) {
     const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, G::kLds);
     if (err != hipSuccess) return fail(HKMOE_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(err));
     attr_set[dev] = true;
   }
-  hk_launch(kern, dim3(grid), dim3(kThreads), lds, stream, p);
+  hk_launch(kern, dim3(grid), dim3(G::kThreads), G::kLds, stream, p);
   return check_launch("gemm_fp8_narrow");
 }
 
-template <Epi EPI>
-int launch_narrow(GemmParams p, hipStream_t stream, int grid) {
+// Prefetch depth: 8 K steps where they divide the step count (and, with block
+// scales, an item's scales fit beside that ring: 64 steps), else 4, the last
+// group padded with empty steps.
+template <Epi EPI, Scale SC, int NW, int ROWS>
+int launch_narrow_p(const GemmParams& p, hipStream_t stream, int grid) {
+  const int k_steps = p.K / kBK;
+  if (k_steps % 8 == 0 && k_steps <= NarrowGeo<SC, 8, NW, ROWS>::kMaxSteps)
+    return launch_narrow_v<EPI, SC, 8, NW, ROWS, false>(p, stream, grid);
+  return launch_narrow_v<EPI, SC, 4, NW, ROWS, true>(p, stream, grid);
+}
+
+// How the narrow path shares a grouped GEMM.  count: device count of narrow M
+// tiles (null: no narrow path, the 256x256 kernel takes every tile).  active ==
+// 0: the 256x256 kernel on the other tiles; yield_from > 0 leaves CUs >=
+// yield_from to the narrow kernel when it has work, < 0 is the late-join launch
+// of `grid` workgroups.  active > 0: the narrow kernel on exactly the narrow
+// tiles, on `grid` workgroups, `active` of them while 256x256 tiles exist;
+// max_rows > 0: nothing runs beside it, and no segment has more rows.
+struct NarrowPart {
+  const int32_t* count = nullptr;
+  int yield_from = 0, active = 0, grid = 0;
+  int64_t max_rows = 0;
+};
+
+template <Epi EPI, Scale SC>
+int launch_narrow(GemmParams p, hipStream_t stream, const NarrowPart& part) {
   p.a_bytes = static_cast<uint32_t>(std::min<int64_t>(p.a_rows * p.K, 0xffffffffll));
-  switch (narrow_depth(p.K / kBK)) {
-    case 8: return launch_narrow_p<EPI, 8>(p, stream, grid);
-    case 4: return launch_narrow_p<EPI, 4>(p, stream, grid);
-    case 2: return launch_narrow_p<EPI, 2>(p, stream, grid);
-    default: return fail(HKMOE_ERR_INVALID_ARGUMENT, "narrow GEMM: K=%d has an odd number of 128 steps", p.K);
+  const int grid = part.grid > 0 ? part.grid : part.active;
+  if constexpr (EPI != Epi::kSiluQuant) {
+    // Alone on the chip, items of half a tile (4 waves): finer last rounds, and
+    // twice the items for shapes with fewer tiles than CUs.  Layer, 8 / 4 waves:
+    // E=128 H=4096 I=1536 MX T=48 388 / 368 us, E=8 H=4096 I=14336 per-tensor T=29 264 /
+    // 246 us.  With at most 16 rows per segment and no more than half a CU per tile, quarters
+    // (2 waves, four workgroups per CU): E=128 T=1 second GEMM 24.6 -> 12.8 us; with more
+    // tiles their fixed cost per item loses (T=4 49 / 41 us).
+    const int64_t tiles = std::min<int64_t>(p.num_experts, p.rows) * p.n_tiles;  // at most
+    if (part.max_rows > 0 && part.max_rows <= 16 && tiles <= grid / 2)
+      return launch_narrow_p<EPI, SC, 2, 16>(p, stream, 4 * grid);
+    if (part.max_rows > 0) return launch_narrow_p<EPI, SC, 4, kNarrowRows>(p, stream, grid);
   }
+  return launch_narrow_p<EPI, SC, 8, kNarrowRows>(p, stream, grid);
 }
 
 // Narrow path settings, read once from the environment:
@@ -513,6 +537,9 @@ int scratch_ptr(void** out) {
   *out = g_scratch_ptr[dev];
   return HKMOE_OK;
 }
+
+// K step counts that hkmoe_grouped_gemm{1,2}_part take for part 1.
+bool narrow_part_steps(int k_steps) { return k_steps % 2 == 0 && k_steps <= 64; }
 
 // Workgroups the narrow kernels may take while 256x256 tiles exist: at most
 // three quarters of the CUs, so the first 256x256 GEMM keeps at least a quarter
@@ -695,10 +722,6 @@ int hkmoe_scatter(const int32_t* topk_idx, int64_t num_tokens, int32_t num_exper
   return check_launch("scatter_kernel");
 }
 
-// narrow_cnt: skip (wide kernel) the list's last *narrow_cnt M tiles, and with
-// yield_from > 0 leave CUs >= yield_from to the narrow kernel when it has work;
-// narrow_active > 0: run the narrow kernel on exactly those tiles instead (one
-// workgroup per CU; narrow_active of them while 256x256 tiles exist).
 static int grouped_gemm1_impl(const void* x, const float* x_scale, const int32_t* gather,
                               int32_t gather_div, int64_t x_rows, const void* w13, const float* w13_scale,
                               const int32_t* offsets, const int32_t* mtile_offsets,
@@ -706,8 +729,7 @@ static int grouped_gemm1_impl(const void* x, const float* x_scale, const int32_t
                               int32_t num_experts, int32_t hidden, int32_t inter, int scale_mode,
                               int w_layout, int out_format, void* h, float* h_aux,
                               int32_t* tile_counters, hkmoe_stream_t stream,
-                              const int32_t* narrow_cnt, int yield_from, int narrow_active,
-                              int narrow_grid = 0) {
+                              const NarrowPart& part) {
   HK_REQUIRE(w13 && w13_scale && offsets && mtile_offsets, "grouped_gemm1: null pointer");
   HK_REQUIRE(rows == 0 || (x && x_scale && h), "grouped_gemm1: null pointer");
   HK_REQUIRE(num_experts >= 1 && num_experts <= kMaxExperts, "grouped_gemm1: bad E=%d", num_experts);
@@ -751,17 +773,21 @@ static int grouped_gemm1_impl(const void* x, const float* x_scale, const int32_t
   p.mtile_list = mtile_list;
   p.blk_m_log2 = block_m_log2(1);  // 2 x 16 tile blocks by default
   p.tile_ctr = tile_counters;
-  p.narrow_cnt = narrow_cnt;
-  p.yield_from = yield_from;
-  p.narrow_active = narrow_active;
+  p.narrow_cnt = part.count;
+  p.yield_from = part.yield_from;
+  p.narrow_active = part.active;
   auto s = static_cast<hipStream_t>(stream);
-  if (narrow_active > 0) {
-    if (scale_mode != HKMOE_SCALE_BLOCK || out_format != HKMOE_E4M3 || narrow_cnt == nullptr ||
-        mtile_list == nullptr || tile_counters == nullptr)
-      return fail(HKMOE_ERR_INVALID_ARGUMENT, "grouped_gemm1: the narrow kernel needs block scales, "
-                                              "e4m3 output, the M-tile list and an item counter");
+  if (part.active > 0) {
+    if (part.count == nullptr || mtile_list == nullptr || tile_counters == nullptr ||
+        (scale_mode == HKMOE_SCALE_BLOCK && out_format != HKMOE_E4M3))
+      return fail(HKMOE_ERR_INVALID_ARGUMENT, "grouped_gemm1: the narrow kernel needs the M-tile list, an item "
+                                              "counter and, with block scales, e4m3 output");
+    if (scale_mode == HKMOE_SCALE_TENSOR) {
+      p.amax = h_aux;
+      return launch_narrow<Epi::kSiluBf16, Scale::kTensor>(p, s, part);
+    }
     p.c_scale = h_aux;
-    return launch_narrow<Epi::kSiluQuant>(p, s, narrow_grid > 0 ? narrow_grid : narrow_active);
+    return launch_narrow<Epi::kSiluQuant, Scale::kBlock>(p, s, part);
   }
   if (scale_mode == HKMOE_SCALE_TENSOR) {
     p.amax = h_aux;
@@ -769,7 +795,7 @@ static int grouped_gemm1_impl(const void* x, const float* x_scale, const int32_t
   }
   if (out_format == HKMOE_E4M3) {
     p.c_scale = h_aux;
-    return launch_gemm<Epi::kSiluQuant, Scale::kBlock>(p, s, yield_from < 0 ? narrow_grid : 0);
+    return launch_gemm<Epi::kSiluQuant, Scale::kBlock>(p, s, part.yield_from < 0 ? part.grid : 0);
   }
   return launch_gemm<Epi::kSiluBf16, Scale::kBlock>(p, s);
 }
@@ -783,7 +809,7 @@ int hkmoe_grouped_gemm1(const void* x, const float* x_scale, const int32_t* gath
                         int32_t* tile_counters, hkmoe_stream_t stream) {
   return grouped_gemm1_impl(x, x_scale, gather, gather_div, x_rows, w13, w13_scale, offsets,
                             mtile_offsets, mtile_list, rows, num_experts, hidden, inter, scale_mode,
-                            w_layout, out_format, h, h_aux, tile_counters, stream, nullptr, 0, 0);
+                            w_layout, out_format, h, h_aux, tile_counters, stream, NarrowPart{});
 }
 
 int hkmoe_requant(const void* h, int64_t rows, int32_t inter, int scale_mode, const float* amax,
@@ -815,8 +841,7 @@ static int grouped_gemm2_impl(const void* hq, const float* hs, const void* w2, c
                               const int32_t* mtile_list, int64_t rows,
                               int32_t num_experts, int32_t hidden, int32_t inter, int scale_mode,
                               int w_layout, void* y, int32_t* tile_counters, hkmoe_stream_t stream,
-                              const int32_t* narrow_cnt, int yield_from, int narrow_active,
-                              int narrow_grid = 0) {
+                              const NarrowPart& part) {
   HK_REQUIRE(w2 && w2_scale && offsets && mtile_offsets, "grouped_gemm2: null pointer");
   HK_REQUIRE(rows == 0 || (hq && hs && y), "grouped_gemm2: null pointer");
   HK_REQUIRE(num_experts >= 1 && num_experts <= kMaxExperts, "grouped_gemm2: bad E=%d", num_experts);
@@ -852,16 +877,16 @@ static int grouped_gemm2_impl(const void* hq, const float* hs, const void* w2, c
   p.mtile_list = mtile_list;
   p.blk_m_log2 = block_m_log2(2);  // 2 x 16 tile blocks by default
   p.tile_ctr = tile_counters;
-  p.narrow_cnt = narrow_cnt;
-  p.yield_from = yield_from;
-  p.narrow_active = narrow_active;
+  p.narrow_cnt = part.count;
+  p.yield_from = part.yield_from;
+  p.narrow_active = part.active;
   auto s = static_cast<hipStream_t>(stream);
-  if (narrow_active > 0) {
-    if (scale_mode != HKMOE_SCALE_BLOCK || narrow_cnt == nullptr || mtile_list == nullptr ||
-        tile_counters == nullptr)
-      return fail(HKMOE_ERR_INVALID_ARGUMENT, "grouped_gemm2: the narrow kernel needs block scales, "
-                                              "the M-tile list and an item counter");
-    return launch_narrow<Epi::kStoreBf16>(p, s, narrow_grid > 0 ? narrow_grid : narrow_active);
+  if (part.active > 0) {
+    if (part.count == nullptr || mtile_list == nullptr || tile_counters == nullptr)
+      return fail(HKMOE_ERR_INVALID_ARGUMENT, "grouped_gemm2: the narrow kernel needs the M-tile list and an "
+                                              "item counter");
+    return scale_mode == HKMOE_SCALE_BLOCK ? launch_narrow<Epi::kStoreBf16, Scale::kBlock>(p, s, part)
+                                           : launch_narrow<Epi::kStoreBf16, Scale::kTensor>(p, s, part);
   }
   return scale_mode == HKMOE_SCALE_BLOCK ? launch_gemm<Epi::kStoreBf16, Scale::kBlock>(p, s)
                                          : launch_gemm<Epi::kStoreBf16, Scale::kTensor>(p, s);
@@ -873,7 +898,7 @@ int hkmoe_grouped_gemm2(const void* hq, const float* hs, const void* w2, const f
                         int32_t num_experts, int32_t hidden, int32_t inter, int scale_mode,
                         int w_layout, void* y, int32_t* tile_counters, hkmoe_stream_t stream) {
   return grouped_gemm2_impl(hq, hs, w2, w2_scale, offsets, mtile_offsets, mtile_list, rows, num_experts,
-                            hidden, inter, scale_mode, w_layout, y, tile_counters, stream, nullptr, 0, 0);
+                            hidden, inter, scale_mode, w_layout, y, tile_counters, stream, NarrowPart{});
 }
 
 int hkmoe_grouped_gemm1_part(const void* x, const float* x_scale, const int32_t* gather,
@@ -885,18 +910,18 @@ int hkmoe_grouped_gemm1_part(const void* x, const float* x_scale, const int32_t*
   HK_REQUIRE(narrow_info && mtile_list, "grouped_gemm1_part: needs narrow_info and mtile_list");
   HK_REQUIRE(part == 0 || part == 1, "grouped_gemm1_part: part=%d must be 0 (wide) or 1 (narrow)", part);
   HK_REQUIRE(grid >= 0 && grid <= 65536, "grouped_gemm1_part: bad grid %d", grid);
-  HK_REQUIRE(part == 0 || narrow_depth(hidden / kBK) > 0,
+  HK_REQUIRE(part == 0 || narrow_part_steps(hidden / kBK),
              "grouped_gemm1_part: the narrow kernel needs an even number of at most 64 128-wide K steps (H=%d)", hidden);
   if (part == 1) {
     // the narrow kernel's item counter: narrow_info[1], zeroed by hkmoe_expert_offsets_narrow
     return grouped_gemm1_impl(x, x_scale, gather, gather_div, x_rows, w13, w13_scale, offsets, mtile_offsets,
                               mtile_list, rows, num_experts, hidden, inter, HKMOE_SCALE_BLOCK, w_layout,
-                              HKMOE_E4M3, hq, hs, const_cast<int32_t*>(narrow_info) + 1, stream, narrow_info, 0,
-                              grid > 0 ? grid : device_cus(), device_cus());
+                              HKMOE_E4M3, hq, hs, const_cast<int32_t*>(narrow_info) + 1, stream,
+                              NarrowPart{narrow_info, 0, grid > 0 ? grid : device_cus(), device_cus()});
   }
   return grouped_gemm1_impl(x, x_scale, gather, gather_div, x_rows, w13, w13_scale, offsets, mtile_offsets,
                             mtile_list, rows, num_experts, hidden, inter, HKMOE_SCALE_BLOCK, w_layout, HKMOE_E4M3,
-                            hq, hs, tile_counters, stream, narrow_info, grid, 0);
+                            hq, hs, tile_counters, stream, NarrowPart{narrow_info, grid});
 }
 
 int hkmoe_grouped_gemm2_part(const void* hq, const float* hs, const void* w2, const float* w2_scale,
@@ -907,14 +932,14 @@ int hkmoe_grouped_gemm2_part(const void* hq, const float* hs, const void* w2, co
   HK_REQUIRE(narrow_info && mtile_list, "grouped_gemm2_part: needs narrow_info and mtile_list");
   HK_REQUIRE(part == 0 || part == 1, "grouped_gemm2_part: part=%d must be 0 (wide) or 1 (narrow)", part);
   HK_REQUIRE(grid >= 0 && grid <= 65536, "grouped_gemm2_part: bad grid %d", grid);
-  HK_REQUIRE(part == 0 || narrow_depth(inter / kBK) > 0,
+  HK_REQUIRE(part == 0 || narrow_part_steps(inter / kBK),
              "grouped_gemm2_part: the narrow kernel needs an even number of at most 64 128-wide K steps (I=%d)", inter);
   // the narrow kernel's item counter: narrow_info[2], zeroed by hkmoe_expert_offsets_narrow
   return grouped_gemm2_impl(hq, hs, w2, w2_scale, offsets, mtile_offsets, mtile_list, rows, num_experts, hidden,
                             inter, HKMOE_SCALE_BLOCK, w_layout, y,
                             part == 1 ? const_cast<int32_t*>(narrow_info) + 2 : tile_counters, stream,
-                            narrow_info, part == 0 ? grid : 0, part == 1 ? (grid > 0 ? grid : device_cus()) : 0,
-                            part == 1 ? device_cus() : 0);
+                            part == 0 ? NarrowPart{narrow_info, grid}
+                                      : NarrowPart{narrow_info, 0, grid > 0 ? grid : device_cus(), device_cus()});
 }
 
 int hkmoe_pack_weights(const void* w, int64_t num_experts, int64_t n, int64_t k, int32_t gate_up,
@@ -1041,6 +1066,146 @@ size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t
   return carve(nullptr, num_tokens, num_experts, top_k, hidden, inter, scale_mode).bytes;
 }
 
+// Which schedule the layer's experts take.  Experts of at most
+// HKMOE_NARROW_MAX rows go to the weight-streaming narrow kernels, in one of two ways:
+//   seq: up to 2*max_rows rows per expert on average (T*k <= 2*E*max_rows) the
+//     small experts' weight stream dominates: the narrow kernels run on `stream`
+//     after the 256x256 ones, each on every CU, without the fork to the auxiliary stream and the join
+//     back (about 20 us of cross-stream latency).  Measured on the block-scaled config-3
+//     shape (H=7168, I=2048, E=256, k=8): T=512 / 1024 / 2048 / 4096 run 26 / 21 /
+//     13 / 4% faster on one stream, T=6144 / 8192 10 / 8% slower;
+//   aux: on the library's auxiliary stream, beside the 256x256 kernels of the
+//     larger experts on `stream`.  Not with per-tensor scales, whose
+//     requantisation between the GEMMs needs both parts of GEMM 1.
+struct NarrowPlan {
+  NarrowConfig cfg{};
+  bool seq = false;
+  AuxStreams* aux = nullptr;
+  std::unique_lock<std::mutex> lock;  // held while the fork / join is enqueued
+  bool on() const { return seq || aux != nullptr; }
+};
+
+// aux_ok: the layer may use the auxiliary stream (else layers that need it run
+// the 256x256 kernels alone).  tuned: block scales and at most 64 K steps, an even
+// number, in both GEMMs; the lines above were measured there.  For the rest
+// (per-tensor and MX scales, other step counts) the 256x256 kernels lose less to
+// small experts, and two narrow launches that find none cost 8 us: they
+// take the narrow path
+//   with at most max_rows tokens (every expert is narrow): E=8 H=4096 I=14336
+//     per-tensor T=29 328 -> 246 us, E=128 H=4096 I=1536 MX T=48 454 -> 368 us;
+//   and from 256 experts on, where skewed routing leaves many small ones beside a few
+//     large: H=7168 I=2048 per-tensor T=1700 1397 -> 1309 us, MX T=3001 1865 -> 1802 us,
+//     T=8192 3631 -> 3312 us (uniform routing, no small expert: 2211 / 2216 us).  With
+//     fewer experts the two kernels one after the other lose what the smaller one
+//     gains: E=8 per-tensor T=200 skewed 350 / 411 us, E=128 MX T=600 429 / 469 us.
+static int plan_narrow(int64_t num_tokens, int64_t rows, int32_t num_experts, bool tuned, bool aux_ok, hipStream_t s,
+                       NarrowPlan* plan) {
+  plan->cfg = narrow_config();
+  const int64_t max_rows = plan->cfg.max_rows;
+  if (plan->cfg.cus <= 0 || max_rows <= 0) return HKMOE_OK;
+  if (!tuned && num_tokens > max_rows && num_experts < 256) return HKMOE_OK;
+  plan->seq = num_tokens <= max_rows || rows <= 2 * num_experts * max_rows;
+  if (plan->seq || !aux_ok) return HKMOE_OK;
+  HK_TRY(get_aux(s, &plan->aux));
+  if (plan->aux) plan->lock = std::unique_lock<std::mutex>(g_aux_mu);
+  return HKMOE_OK;
+}
+
+// Routing, permutation, both grouped GEMMs and the combine, enqueued by `plan`.
+// gemm1 / gemm2(part, counters, stream) launch one grouped GEMM; prep() what the
+// 256x256 kernel of GEMM 1 needs beyond the routing tables; mid() what comes between
+// the GEMMs.
+extern "C++" {
+template <typename Prep, typename G1, typename Mid, typename G2>
+int moe_enqueue(const float* logits, const MoeWorkspace& w, int64_t num_tokens, int32_t num_experts, int32_t top_k,
+                int32_t hidden, void* out, hipStream_t s, NarrowPlan& plan, Prep prep, G1 gemm1, Mid mid, G2 gemm2) {
+  const NarrowConfig& nc = plan.cfg;
+  const int cus = device_cus();
+  TimedCall timed_call;
+  t_role = HKMOE_TIMING_ROUTE;
+  HK_TRY(hkmoe_route_topk(logits, num_tokens, num_experts, top_k, w.topk_idx, w.topk_w, w.block_counts, s));
+  t_role = HKMOE_TIMING_OFFSETS;
+  HK_TRY(launch_expert_offsets(w.block_counts, num_tokens, num_experts, w.counts, w.offsets, w.block_base,
+                               w.mtile_offsets, w.mtile_list, w.amax, w.tile_ctr, plan.on() ? nc.max_rows : 0,
+                               plan.on() ? w.narrow_info : nullptr, s));
+  t_role = HKMOE_TIMING_SCATTER;
+  HK_TRY(hkmoe_scatter(w.topk_idx, num_tokens, num_experts, top_k, w.offsets, w.block_base, w.perm, w.inv_perm,
+                       nullptr, nullptr, hidden, HKMOE_SCALE_TENSOR, nullptr, nullptr, s));
+  if (plan.seq) {
+    // each 256x256 GEMM keeps every CU and skips the narrow experts' tiles; each
+    // narrow GEMM then runs its items on every CU.  A token's k experts are
+    // distinct, so no expert has more than T rows: with T <= max_rows every
+    // expert is narrow, and the 256x256 GEMMs, which would find no tile, are not
+    // launched.
+    const bool wide = num_tokens > nc.max_rows;
+    const NarrowPart skip{w.narrow_info}, narrow{w.narrow_info, 0, cus, cus, std::min<int64_t>(num_tokens, nc.max_rows)};
+    if (wide) {
+      HK_TRY(prep());
+      t_role = HKMOE_TIMING_GEMM1;
+      HK_TRY(gemm1(skip, w.tile_ctr, s));
+    }
+    t_role = HKMOE_TIMING_GEMM1_NARROW;
+    HK_TRY(gemm1(narrow, w.narrow_info + 1, s));
+    HK_TRY(mid());
+    t_role = HKMOE_TIMING_GEMM2;
+    if (wide) HK_TRY(gemm2(skip, w.tile_ctr + 8, s));
+    t_role = HKMOE_TIMING_GEMM2_NARROW;
+    HK_TRY(gemm2(narrow, w.narrow_info + 2, s));
+  } else if (AuxStreams* aux = plan.aux) {
+    // fork: both GEMMs of the narrow experts on the auxiliary stream, enqueued
+    // first so that their workgroups find free CUs; join before the combine
+    // (prep() first: beside the narrow kernels its few workgroups would wait for
+    // CUs, 69 against 12 us for the MX words, and the 256x256 GEMM 1 with them)
+    HK_TRY(prep());
+    const int ncus = narrow_cus_limit(nc.cus);
+    // Which workgroups work is decided on the device from narrow_info: with
+    // experts of both kinds the narrow kernels use ncus workgroups and (share)
+    // the first 256x256 GEMM leaves them those CUs; with one kind only, that
+    // kind gets every CU it was launched on.
+    if (hipEventRecord(aux->fork, s) != hipSuccess)
+      return fail(HKMOE_ERR_HIP, "moe_forward: fork event failed");
+    const int yield_from = nc.share ? cus - ncus : 0;  // >= device_cus() / 4
+    if (hipStreamWaitEvent(aux->aux, aux->fork, 0) != hipSuccess)
+      return fail(HKMOE_ERR_HIP, "moe_forward: fork to the auxiliary stream failed");
+    AuxJoin guard{aux, s};
+    // the narrow kernels launch one workgroup per CU: beside 256x256 tiles the
+    // first ncus to start take items, else all of them (decode-like shapes)
+    const NarrowPart narrow{w.narrow_info, 0, ncus, cus};
+    t_role = HKMOE_TIMING_GEMM1_NARROW;
+    HK_TRY(gemm1(narrow, w.narrow_info + 1, aux->aux));
+    t_role = HKMOE_TIMING_GEMM2_NARROW;
+    HK_TRY(gemm2(narrow, w.narrow_info + 2, aux->aux));
+    // share == 2: once the narrow GEMMs are done, their CUs join the first 256x256
+    // GEMM's tile queues (a second launch of it on the auxiliary stream, which
+    // takes whatever tiles are left); the second 256x256 GEMM then waits for both.
+    const bool late_join = nc.share == 2;
+    t_role = HKMOE_TIMING_GEMM1_JOIN;
+    if (late_join) HK_TRY(gemm1(NarrowPart{w.narrow_info, -1, 0, ncus}, w.tile_ctr, aux->aux));
+    if (hipEventRecord(aux->join, aux->aux) != hipSuccess)
+      return fail(HKMOE_ERR_HIP, "moe_forward: join event failed");
+    t_role = HKMOE_TIMING_GEMM1;
+    HK_TRY(gemm1(NarrowPart{w.narrow_info, yield_from}, w.tile_ctr, s));
+    if (late_join && hipStreamWaitEvent(s, aux->join, 0) != hipSuccess)
+      return fail(HKMOE_ERR_HIP, "moe_forward: join of the auxiliary stream failed");
+    t_role = HKMOE_TIMING_GEMM2;
+    HK_TRY(gemm2(NarrowPart{w.narrow_info}, w.tile_ctr + 8, s));
+    if (!late_join && hipStreamWaitEvent(s, aux->join, 0) != hipSuccess)
+      return fail(HKMOE_ERR_HIP, "moe_forward: join of the auxiliary stream failed");
+    guard.armed = false;  // joined above
+    plan.lock.unlock();
+  } else {
+    HK_TRY(prep());
+    t_role = HKMOE_TIMING_GEMM1;
+    HK_TRY(gemm1(NarrowPart{}, w.tile_ctr, s));
+    HK_TRY(mid());
+    t_role = HKMOE_TIMING_GEMM2;
+    HK_TRY(gemm2(NarrowPart{}, w.tile_ctr + 8, s));
+  }
+  t_role = HKMOE_TIMING_COMBINE;
+  return hkmoe_combine(w.y, w.topk_w, w.inv_perm, num_tokens, top_k, hidden, out, s);
+}
+}  // extern "C++"
+
 // The layer; aux_ok: the narrow path may fork to the library's auxiliary
 // stream (else every kernel runs on `stream`: the one-stream narrow schedule
 // where it applies, otherwise the 256x256 kernels alone).
@@ -1081,149 +1246,28 @@ static int moe_forward_impl(const void* x_q, const float* x_scale, const float* 
                                hidden, inter, scale_mode);
   const int64_t rows = num_tokens * top_k;
   auto s = static_cast<hipStream_t>(stream);
-  // Narrow path (block scales): experts of at most HKMOE_NARROW_MAX rows go to
-  // the weight-streaming narrow kernels on an auxiliary stream, which run
-  // beside the 256x256 kernels of the larger experts on the main stream.
-  const NarrowConfig nc = narrow_config();
-  const bool narrow_ok = block && nc.cus > 0 && nc.max_rows > 0 && narrow_depth(hidden / kBK) > 0 &&
-                         narrow_depth(inter / kBK) > 0;
-  // Up to 2*max_rows rows per expert on average (T*k <= 2*E*max_rows) the small
-  // experts' weight stream dominates: the narrow kernels then run on `stream`
-  // after the 256x256 ones, each on every CU, instead of on max. 3/4 of them
-  // beside the 256x256 kernels, and without the fork to the auxiliary stream and
-  // the join back (≈20 µs of cross-stream latency).  Measured on the config-3
-  // shape (H=7168, I=2048, E=256, k=8): T=512 / 1024 / 2048 / 4096 run 26 / 21 /
-  // 13 / 4% faster on one stream, T=6144 / 8192 10 / 8% slower.
-  const bool narrow_seq = narrow_ok && rows <= 2 * static_cast<int64_t>(num_experts) * nc.max_rows;
-  // the two-stream schedule needs the auxiliary stream; without it (aux_ok
-  // false) such layers run the 256x256 kernels alone
-  AuxStreams* aux = nullptr;
-  if (aux_ok && narrow_ok && !narrow_seq) HK_TRY(get_aux(s, &aux));
-  std::unique_lock<std::mutex> aux_lock(g_aux_mu, std::defer_lock);
-  if (aux) aux_lock.lock();
-  TimedCall timed_call;
-  t_role = HKMOE_TIMING_ROUTE;
-  HK_TRY(hkmoe_route_topk(logits, num_tokens, num_experts, top_k, w.topk_idx, w.topk_w,
-                          w.block_counts, stream));
-  t_role = HKMOE_TIMING_OFFSETS;
-  HK_TRY(launch_expert_offsets(w.block_counts, num_tokens, num_experts, w.counts, w.offsets,
-                               w.block_base, w.mtile_offsets, w.mtile_list, w.amax, w.tile_ctr,
-                               (aux || narrow_seq) ? nc.max_rows : 0,
-                               (aux || narrow_seq) ? w.narrow_info : nullptr, s));
-  t_role = HKMOE_TIMING_SCATTER;
-  HK_TRY(hkmoe_scatter(w.topk_idx, num_tokens, num_experts, top_k, w.offsets, w.block_base, w.perm,
-                       w.inv_perm, nullptr, nullptr, hidden, scale_mode, nullptr, nullptr, stream));
-  if (narrow_seq) {
-    // one stream: each 256x256 GEMM keeps every CU (yield_from 0) and skips the
-    // narrow experts' tiles; each narrow GEMM then runs its items on every CU.
-    // A token's k experts are distinct, so no expert has more than T rows: with
-    // T <= max_rows every expert is narrow, and the 256x256 GEMMs, which would
-    // find no tile, are not launched.
-    const int ngrid = device_cus();
-    const bool wide = num_tokens > nc.max_rows;
-    t_role = HKMOE_TIMING_GEMM1;
-    if (wide)
-      HK_TRY(grouped_gemm1_impl(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets,
-                                w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter, scale_mode,
-                                w_layout, HKMOE_E4M3, w.hq, w.hs, w.tile_ctr, stream, w.narrow_info, 0, 0));
-    t_role = HKMOE_TIMING_GEMM1_NARROW;
-    HK_TRY(grouped_gemm1_impl(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets,
-                              w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter, scale_mode,
-                              w_layout, HKMOE_E4M3, w.hq, w.hs, w.narrow_info + 1, stream, w.narrow_info, 0,
-                              ngrid, ngrid));
-    t_role = HKMOE_TIMING_GEMM2;
-    if (wide)
-      HK_TRY(grouped_gemm2_impl(w.hq, w.hs, w2, w2_scale, w.offsets, w.mtile_offsets, w.mtile_list, rows,
-                                num_experts, hidden, inter, scale_mode, w_layout, w.y, w.tile_ctr + 8, stream,
-                                w.narrow_info, 0, 0));
-    t_role = HKMOE_TIMING_GEMM2_NARROW;
-    HK_TRY(grouped_gemm2_impl(w.hq, w.hs, w2, w2_scale, w.offsets, w.mtile_offsets, w.mtile_list, rows,
-                              num_experts, hidden, inter, scale_mode, w_layout, w.y, w.narrow_info + 2, stream,
-                              w.narrow_info, 0, ngrid, ngrid));
-    t_role = HKMOE_TIMING_COMBINE;
-    HK_TRY(hkmoe_combine(w.y, w.topk_w, w.inv_perm, num_tokens, top_k, hidden, out, stream));
-    return HKMOE_OK;
-  }
-  if (aux) {
-    // fork: both GEMMs of the narrow experts on the auxiliary stream, enqueued
-    // first so that their workgroups find free CUs; join before the combine
-    const int ncus = narrow_cus_limit(nc.cus);
-    // Which workgroups work is decided on the device from narrow_info: with
-    // experts of both kinds the narrow kernels use ncus workgroups and (share)
-    // the first 256x256 GEMM leaves them those CUs; with one kind only, that
-    // kind gets every CU it was launched on.
-    if (hipEventRecord(aux->fork, s) != hipSuccess)
-      return fail(HKMOE_ERR_HIP, "moe_forward: fork event failed");
-    const int yield_from = nc.share ? device_cus() - ncus : 0;  // >= device_cus() / 4
-    if (hipStreamWaitEvent(aux->aux, aux->fork, 0) != hipSuccess)
-      return fail(HKMOE_ERR_HIP, "moe_forward: fork to the auxiliary stream failed");
-    AuxJoin guard{aux, s};
-    // the narrow kernels launch one workgroup per CU: beside 256x256 tiles the
-    // first ncus to start take items, else all of them (decode-like shapes)
-    const int ngrid = device_cus();
-    t_role = HKMOE_TIMING_GEMM1_NARROW;
-    HK_TRY(grouped_gemm1_impl(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets,
-                              w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter, scale_mode,
-                              w_layout, HKMOE_E4M3, w.hq, w.hs, w.narrow_info + 1, aux->aux,
-                              w.narrow_info, 0, ncus, ngrid));
-    t_role = HKMOE_TIMING_GEMM2_NARROW;
-    HK_TRY(grouped_gemm2_impl(w.hq, w.hs, w2, w2_scale, w.offsets, w.mtile_offsets, w.mtile_list, rows,
-                              num_experts, hidden, inter, scale_mode, w_layout, w.y, w.narrow_info + 2,
-                              aux->aux, w.narrow_info, 0, ncus, ngrid));
-    // share == 2: once the narrow GEMMs are done, their CUs join the first 256x256
-    // GEMM's tile queues (a second launch of it on the auxiliary stream, which
-    // takes whatever tiles are left); the second 256x256 GEMM then waits for both.
-    // (Shapes with rows <= 2 * E * max_rows took the one-stream path above.)
-    const bool late_join = nc.share == 2;
-    t_role = HKMOE_TIMING_GEMM1_JOIN;
-    if (late_join)
-      HK_TRY(grouped_gemm1_impl(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets,
-                                w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter, scale_mode,
-                                w_layout, HKMOE_E4M3, w.hq, w.hs, w.tile_ctr, aux->aux, w.narrow_info,
-                                -1, 0, ncus));
-    if (hipEventRecord(aux->join, aux->aux) != hipSuccess)
-      return fail(HKMOE_ERR_HIP, "moe_forward: join event failed");
-    t_role = HKMOE_TIMING_GEMM1;
-    HK_TRY(grouped_gemm1_impl(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets,
-                              w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter, scale_mode,
-                              w_layout, HKMOE_E4M3, w.hq, w.hs, w.tile_ctr, stream, w.narrow_info,
-                              yield_from, 0));
-    if (late_join && hipStreamWaitEvent(s, aux->join, 0) != hipSuccess)
-      return fail(HKMOE_ERR_HIP, "moe_forward: join of the auxiliary stream failed");
-    t_role = HKMOE_TIMING_GEMM2;
-    HK_TRY(grouped_gemm2_impl(w.hq, w.hs, w2, w2_scale, w.offsets, w.mtile_offsets, w.mtile_list, rows,
-                              num_experts, hidden, inter, scale_mode, w_layout, w.y, w.tile_ctr + 8,
-                              stream, w.narrow_info, 0, 0));
-    if (!late_join && hipStreamWaitEvent(s, aux->join, 0) != hipSuccess)
-      return fail(HKMOE_ERR_HIP, "moe_forward: join of the auxiliary stream failed");
-    guard.armed = false;  // joined above
-    aux_lock.unlock();
-    t_role = HKMOE_TIMING_COMBINE;
-    HK_TRY(hkmoe_combine(w.y, w.topk_w, w.inv_perm, num_tokens, top_k, hidden, out, stream));
-    return HKMOE_OK;
-  }
-  if (block) {
-    // GEMM 1 reads token rows through perm and writes the requantised e4m3
-    // intermediate and its 1x128 group scales directly.
-    t_role = HKMOE_TIMING_GEMM1;
-    HK_TRY(hkmoe_grouped_gemm1(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets,
-                               w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter,
-                               scale_mode, w_layout, HKMOE_E4M3, w.hq, w.hs, w.tile_ctr, stream));
-  } else {
-    t_role = HKMOE_TIMING_GEMM1;
-    HK_TRY(hkmoe_grouped_gemm1(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets,
-                               w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter,
-                               scale_mode, w_layout, HKMOE_BF16, w.h, w.amax, w.tile_ctr, stream));
-    t_role = HKMOE_TIMING_REQUANT;
-    HK_TRY(hkmoe_requant(w.h, rows, inter, scale_mode, w.amax, w.hq, w.hs, stream));
-  }
-  t_role = HKMOE_TIMING_GEMM2;
-  HK_TRY(hkmoe_grouped_gemm2(w.hq, w.hs, w2, w2_scale, w.offsets, w.mtile_offsets, w.mtile_list,
-                             rows, num_experts, hidden, inter, scale_mode, w_layout, w.y,
-                             w.tile_ctr + 8, stream));
-  t_role = HKMOE_TIMING_COMBINE;
-  HK_TRY(hkmoe_combine(w.y, w.topk_w, w.inv_perm, num_tokens, top_k, hidden, out, stream));
-  return HKMOE_OK;
+  NarrowPlan plan;
+  const bool tuned = block && narrow_part_steps(hidden / kBK) && narrow_part_steps(inter / kBK);
+  HK_TRY(plan_narrow(num_tokens, rows, num_experts, tuned, aux_ok && block, s, &plan));
+  return moe_enqueue(
+      logits, w, num_tokens, num_experts, top_k, hidden, out, s, plan, [] { return HKMOE_OK; },
+      // GEMM 1 reads token rows through perm; with block scales it writes the
+      // requantised e4m3 intermediate and its 1x128 group scales directly
+      [&](const NarrowPart& part, int32_t* ctr, hipStream_t st) {
+        return grouped_gemm1_impl(x_q, x_scale, w.perm, top_k, num_tokens, w13, w13_scale, w.offsets, w.mtile_offsets,
+                                  w.mtile_list, rows, num_experts, hidden, inter, scale_mode, w_layout,
+                                  block ? HKMOE_E4M3 : HKMOE_BF16, block ? static_cast<void*>(w.hq) : w.h,
+                                  block ? w.hs : w.amax, ctr, st, part);
+      },
+      [&] {
+        if (block) return static_cast<int>(HKMOE_OK);
+        t_role = HKMOE_TIMING_REQUANT;
+        return hkmoe_requant(w.h, rows, inter, scale_mode, w.amax, w.hq, w.hs, s);
+      },
+      [&](const NarrowPart& part, int32_t* ctr, hipStream_t st) {
+        return grouped_gemm2_impl(w.hq, w.hs, w2, w2_scale, w.offsets, w.mtile_offsets, w.mtile_list, rows,
+                                  num_experts, hidden, inter, scale_mode, w_layout, w.y, ctr, st, part);
+      });
 }
 
 int hkmoe_moe_forward(const void* x_q, const float* x_scale, const float* logits, const void* w13,
@@ -1394,11 +1438,14 @@ int hkmoe_mx_gather_scales(const void* s, int64_t x_rows, int32_t k, const int32
   return check_launch("mx_gather_words_kernel");
 }
 
-int hkmoe_grouped_gemm1_mx(const void* x, const void* x_words, const int32_t* gather, int32_t gather_div,
-                           int64_t x_rows, const void* w13, const void* w13_words, const int32_t* offsets,
-                           const int32_t* mtile_offsets, const int32_t* mtile_list, int64_t rows,
-                           int32_t num_experts, int32_t hidden, int32_t inter, int w_layout, int out_format,
-                           void* h, void* h_words, int32_t* tile_counters, hkmoe_stream_t stream) {
+// x_words: the tile-aligned words, or for the narrow kernel (part.active > 0)
+// the rows' own exponent bytes [x_rows, H/32].
+static int grouped_gemm1_mx_impl(const void* x, const void* x_words, const int32_t* gather, int32_t gather_div,
+                                 int64_t x_rows, const void* w13, const void* w13_words, const int32_t* offsets,
+                                 const int32_t* mtile_offsets, const int32_t* mtile_list, int64_t rows,
+                                 int32_t num_experts, int32_t hidden, int32_t inter, int w_layout, int out_format,
+                                 void* h, void* h_words, int32_t* tile_counters, hkmoe_stream_t stream,
+                                 const NarrowPart& part) {
   HK_REQUIRE(w13 && w13_words && offsets && mtile_offsets, "grouped_gemm1_mx: null pointer");
   HK_REQUIRE(rows == 0 || (x && x_words && h), "grouped_gemm1_mx: null pointer");
   HK_REQUIRE(num_experts >= 1 && num_experts <= kMaxExperts, "grouped_gemm1_mx: bad E=%d", num_experts);
@@ -1443,15 +1490,34 @@ int hkmoe_grouped_gemm1_mx(const void* x, const void* x_words, const int32_t* ga
   p.mtile_list = mtile_list;
   p.blk_m_log2 = block_m_log2(1);  // 2 x 16 tile blocks by default
   p.tile_ctr = tile_counters;
+  p.narrow_cnt = part.count;
+  p.yield_from = part.yield_from;
+  p.narrow_active = part.active;
   auto st = static_cast<hipStream_t>(stream);
-  return out_format == HKMOE_E4M3 ? launch_gemm<Epi::kSiluMx, Scale::kMX>(p, st)
-                                  : launch_gemm<Epi::kSiluBf16, Scale::kMX>(p, st);
+  if (part.active > 0) {
+    p.as_rs = hidden / kGroup;  // one dword of exponents per row and K step, row-major
+    p.as_ks = 1;
+    return launch_narrow<Epi::kSiluMx, Scale::kMX>(p, st, part);
+  }
+  const int grid = part.yield_from < 0 ? part.grid : 0;
+  return out_format == HKMOE_E4M3 ? launch_gemm<Epi::kSiluMx, Scale::kMX>(p, st, grid)
+                                  : launch_gemm<Epi::kSiluBf16, Scale::kMX>(p, st, grid);
 }
 
-int hkmoe_grouped_gemm2_mx(const void* hq, const void* hq_words, const void* w2, const void* w2_words,
-                           const int32_t* offsets, const int32_t* mtile_offsets, const int32_t* mtile_list,
-                           int64_t rows, int32_t num_experts, int32_t hidden, int32_t inter, int w_layout,
-                           void* y, int32_t* tile_counters, hkmoe_stream_t stream) {
+int hkmoe_grouped_gemm1_mx(const void* x, const void* x_words, const int32_t* gather, int32_t gather_div,
+                           int64_t x_rows, const void* w13, const void* w13_words, const int32_t* offsets,
+                           const int32_t* mtile_offsets, const int32_t* mtile_list, int64_t rows,
+                           int32_t num_experts, int32_t hidden, int32_t inter, int w_layout, int out_format,
+                           void* h, void* h_words, int32_t* tile_counters, hkmoe_stream_t stream) {
+  return grouped_gemm1_mx_impl(x, x_words, gather, gather_div, x_rows, w13, w13_words, offsets, mtile_offsets,
+                               mtile_list, rows, num_experts, hidden, inter, w_layout, out_format, h, h_words,
+                               tile_counters, stream, NarrowPart{});
+}
+
+static int grouped_gemm2_mx_impl(const void* hq, const void* hq_words, const void* w2, const void* w2_words,
+                                 const int32_t* offsets, const int32_t* mtile_offsets, const int32_t* mtile_list,
+                                 int64_t rows, int32_t num_experts, int32_t hidden, int32_t inter, int w_layout,
+                                 void* y, int32_t* tile_counters, hkmoe_stream_t stream, const NarrowPart& part) {
   HK_REQUIRE(w2 && w2_words && offsets && mtile_offsets, "grouped_gemm2_mx: null pointer");
   HK_REQUIRE(rows == 0 || (hq && hq_words && y), "grouped_gemm2_mx: null pointer");
   HK_REQUIRE(num_experts >= 1 && num_experts <= kMaxExperts, "grouped_gemm2_mx: bad E=%d", num_experts);
@@ -1486,7 +1552,24 @@ int hkmoe_grouped_gemm2_mx(const void* hq, const void* hq_words, const void* w2,
   p.mtile_list = mtile_list;
   p.blk_m_log2 = block_m_log2(2);
   p.tile_ctr = tile_counters;
-  return launch_gemm<Epi::kStoreBf16, Scale::kMX>(p, static_cast<hipStream_t>(stream));
+  p.narrow_cnt = part.count;
+  p.yield_from = part.yield_from;
+  p.narrow_active = part.active;
+  auto st = static_cast<hipStream_t>(stream);
+  if (part.active > 0) {
+    p.as_rs = 1;  // one dword of exponents per row and K step, in the M tile's words
+    p.as_ks = ws;
+    return launch_narrow<Epi::kStoreBf16, Scale::kMX>(p, st, part);
+  }
+  return launch_gemm<Epi::kStoreBf16, Scale::kMX>(p, st);
+}
+
+int hkmoe_grouped_gemm2_mx(const void* hq, const void* hq_words, const void* w2, const void* w2_words,
+                           const int32_t* offsets, const int32_t* mtile_offsets, const int32_t* mtile_list,
+                           int64_t rows, int32_t num_experts, int32_t hidden, int32_t inter, int w_layout,
+                           void* y, int32_t* tile_counters, hkmoe_stream_t stream) {
+  return grouped_gemm2_mx_impl(hq, hq_words, w2, w2_words, offsets, mtile_offsets, mtile_list, rows, num_experts,
+                               hidden, inter, w_layout, y, tile_counters, stream, NarrowPart{});
 }
 
 int hkmoe_moe_forward_mx(const void* x_q, const void* x_e8m0, const float* logits, const void* w13,
@@ -1510,6 +1593,8 @@ int hkmoe_moe_forward_mx(const void* x_q, const void* x_e8m0, const float* logit
   HK_REQUIRE(num_tokens * hidden < (1ll << 32) && num_tokens * top_k * inter < (1ll << 32),
              "moe_forward_mx: T*H and T*k*I must be < 2^32 (32-bit buffer offsets)");
   if (num_tokens == 0) return HKMOE_OK;
+  // both the word gather and the narrow kernel read a row's exponents as dwords
+  HK_REQUIRE((reinterpret_cast<uintptr_t>(x_e8m0) & 3) == 0, "mx_gather_scales: exponents must be 4-byte aligned");
   const MoeWorkspace need = carve(nullptr, num_tokens, num_experts, top_k, hidden, inter, HKMOE_SCALE_MX);
   if (workspace == nullptr || workspace_bytes < need.bytes)
     return fail(HKMOE_ERR_WORKSPACE, "moe_forward_mx: workspace of %zu bytes needed, %zu given", need.bytes,
@@ -1518,29 +1603,27 @@ int hkmoe_moe_forward_mx(const void* x_q, const void* x_e8m0, const float* logit
   const MoeWorkspace w = carve(static_cast<uint8_t*>(workspace), num_tokens, num_experts, top_k, hidden,
                                inter, HKMOE_SCALE_MX);
   const int64_t rows = num_tokens * top_k;
-  TimedCall timed_call;
-  t_role = HKMOE_TIMING_ROUTE;
-  HK_TRY(hkmoe_route_topk(logits, num_tokens, num_experts, top_k, w.topk_idx, w.topk_w, w.block_counts, stream));
-  t_role = HKMOE_TIMING_OFFSETS;
-  HK_TRY(hkmoe_expert_offsets(w.block_counts, num_tokens, num_experts, w.counts, w.offsets, w.block_base,
-                              w.mtile_offsets, w.mtile_list, w.amax, w.tile_ctr, stream));
-  t_role = HKMOE_TIMING_SCATTER;
-  HK_TRY(hkmoe_scatter(w.topk_idx, num_tokens, num_experts, top_k, w.offsets, w.block_base, w.perm, w.inv_perm,
-                       nullptr, nullptr, hidden, HKMOE_SCALE_TENSOR, nullptr, nullptr, stream));
-  // token exponents -> tile-aligned words in expert order (x rows stay in place)
-  t_role = HKMOE_TIMING_MX_WORDS;
-  HK_TRY(hkmoe_mx_gather_scales(x_e8m0, num_tokens, hidden, w.perm, top_k, w.offsets, w.mtile_offsets,
-                                num_experts, rows, w.xw, stream));
-  t_role = HKMOE_TIMING_GEMM1;
-  HK_TRY(hkmoe_grouped_gemm1_mx(x_q, w.xw, w.perm, top_k, num_tokens, w13, w13_words, w.offsets, w.mtile_offsets,
-                                w.mtile_list, rows, num_experts, hidden, inter, w_layout, HKMOE_E4M3, w.hq, w.hs,
-                                w.tile_ctr, stream));
-  t_role = HKMOE_TIMING_GEMM2;
-  HK_TRY(hkmoe_grouped_gemm2_mx(w.hq, w.hs, w2, w2_words, w.offsets, w.mtile_offsets, w.mtile_list, rows,
-                                num_experts, hidden, inter, w_layout, w.y, w.tile_ctr + 8, stream));
-  t_role = HKMOE_TIMING_COMBINE;
-  HK_TRY(hkmoe_combine(w.y, w.topk_w, w.inv_perm, num_tokens, top_k, hidden, out, stream));
-  return HKMOE_OK;
+  auto s = static_cast<hipStream_t>(stream);
+  NarrowPlan plan;
+  HK_TRY(plan_narrow(num_tokens, rows, num_experts, false, true, s, &plan));
+  return moe_enqueue(
+      logits, w, num_tokens, num_experts, top_k, hidden, out, s, plan,
+      // token exponents -> tile-aligned words in expert order (x rows stay in place)
+      [&] {
+        t_role = HKMOE_TIMING_MX_WORDS;
+        return hkmoe_mx_gather_scales(x_e8m0, num_tokens, hidden, w.perm, top_k, w.offsets, w.mtile_offsets,
+                                      num_experts, rows, w.xw, s);
+      },
+      [&](const NarrowPart& part, int32_t* ctr, hipStream_t st) {
+        return grouped_gemm1_mx_impl(x_q, part.active > 0 ? x_e8m0 : w.xw, w.perm, top_k, num_tokens, w13, w13_words,
+                                     w.offsets, w.mtile_offsets, w.mtile_list, rows, num_experts, hidden, inter,
+                                     w_layout, HKMOE_E4M3, w.hq, w.hs, ctr, st, part);
+      },
+      [] { return HKMOE_OK; },
+      [&](const NarrowPart& part, int32_t* ctr, hipStream_t st) {
+        return grouped_gemm2_mx_impl(w.hq, w.hs, w2, w2_words, w.offsets, w.mtile_offsets, w.mtile_list, rows,
+                                     num_experts, hidden, inter, w_layout, w.y, ctr, st, part);
+      });
 }
 
 // ---------------------------------------------------------------------------

@@ -612,7 +612,7 @@ __device__ __forceinline__ float row16_max(float v) {
   return v;
 }
 
-__device__ __forceinline__ float max_abs4(const f32x4& v) {
+__device__ __forceinline__ float max_abs4(f32x4 v) {
   return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 
@@ -621,7 +621,7 @@ __device__ __forceinline__ float max_abs4(const f32x4& v) {
 // pairs with x <= 448 sc and x / sc >= 2^-10 it never differed from x / sc) and
 // the packed conversion; a NaN or an infinite scale keeps the division and the
 // software conversion (NaN code 0x7f | sign).
-__device__ __forceinline__ uint32_t quant4(const f32x4& v, float sc, const QuotScale& qs) {
+__device__ __forceinline__ uint32_t quant4(f32x4 v, float sc, const QuotScale& qs) {
   const bool odd = __builtin_isunordered(v.x, v.y) || __builtin_isunordered(v.z, v.w) || __builtin_isinf(sc);
   if (__builtin_expect(odd, 0))
     return f32_to_e4m3(v.x / sc) | (f32_to_e4m3(v.y / sc) << 8) | (f32_to_e4m3(v.z / sc) << 16) |

@@ -281,27 +281,32 @@ int hkmoe_combine(const void* y, const float* topk_w, const int32_t* inv_perm, i
 size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t top_k,
                                 int32_t hidden, int32_t inter, int scale_mode);
 /*
- * Narrow path of hkmoe_moe_forward (block scales only): the experts with
+ * Narrow path of hkmoe_moe_forward and hkmoe_moe_forward_mx: the experts with
  * 1..max_rows rows (max_rows <= 64) go to a weight-streaming grouped GEMM
- * (both GEMMs) that runs on `cus` workgroups on a library-owned auxiliary
- * stream, beside the 256x256 kernels of the larger experts on the caller's
- * stream; the caller's stream waits for it before the combine.  Results are
- * bit-identical with the narrow path on or off.  cus == 0 turns it off; while
- * 256x256 tiles exist the narrow kernels take at most three quarters of the
- * device's CUs, whatever cus asks for (the first wide GEMM keeps the rest);
- * wide_share 1 or 2 runs the first wide GEMM on (CUs - cus) workgroups while
- * narrow experts exist; with 2 the narrow path's CUs also join that GEMM's
- * remaining tiles once both narrow GEMMs are done (a second launch of it on the
- * auxiliary stream), and the second wide GEMM waits for them.  Other values are
- * rejected.  Shapes with T*top_k <= 2*E*max_rows (small experts dominate) use
- * no auxiliary stream: each narrow GEMM runs on the caller's stream after the
- * wide one, on every CU (and wide_share does not apply).
- * It also stays off when H/128 or I/128 is odd or above 64, and for a first call made
- * while the caller's stream is being captured into a graph (the auxiliary
- * stream is created on the first call that is not captured).  Defaults come
- * from HKMOE_NARROW_CUS, HKMOE_NARROW_MAX and HKMOE_NARROW_SHARE in the
- * environment, else 64, 64 and 1 (out-of-range HKMOE_NARROW_SHARE is clamped to 0..2).  Concurrent hkmoe_moe_forward calls on one
- * device enqueue their fork/join one at a time (a mutex).
+ * (both GEMMs), on one of two schedules:
+ *   one stream: each narrow GEMM runs on the caller's stream after the 256x256
+ *     one, on every CU (and wide_share does not apply): shapes with T*top_k <=
+ *     2*E*max_rows, where small experts dominate;
+ *   auxiliary stream (block and MX scales): on `cus` workgroups of a
+ *     library-owned stream, beside the 256x256 kernels of the larger experts on the
+ *     caller's stream, which waits for it before the combine.
+ * Block-scaled layers with an even number of at most 64 128-wide K steps in both
+ * GEMMs (H/128 and I/128) use it at every T; the others (per-tensor and MX scales,
+ * other step counts) with at most max_rows tokens, where every expert is
+ * narrow, or at least 256 experts.  Results are bit-identical with the narrow path
+ * on or off.  cus == 0 turns it off; while 256x256 tiles exist the narrow kernels
+ * take at most three quarters of the device's CUs, whatever cus asks for (the
+ * first wide GEMM keeps the rest); wide_share 1 or 2 runs the first wide GEMM on
+ * (CUs - cus) workgroups while narrow experts exist; with 2 the narrow path's CUs
+ * also join that GEMM's remaining tiles once both narrow GEMMs are done (a second
+ * launch of it on the auxiliary stream), and the second wide GEMM waits for
+ * them.  Other values are rejected.
+ * The auxiliary schedule stays off for a first call made while the caller's
+ * stream is being captured into a graph (the auxiliary stream is created on the
+ * first call that is not captured).  Defaults come from HKMOE_NARROW_CUS,
+ * HKMOE_NARROW_MAX and HKMOE_NARROW_SHARE in the environment, else 64, 64 and 1
+ * (out-of-range HKMOE_NARROW_SHARE is clamped to 0..2).  Concurrent layer calls on
+ * one device enqueue their fork/join one at a time (a mutex).
  * No reference counterpart: the reference has no grouped GEMM.
  */
 int hkmoe_set_narrow(int32_t cus, int32_t max_rows, int32_t wide_share);
