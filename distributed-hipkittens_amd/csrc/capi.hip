@@ -1116,6 +1116,20 @@ static int plan_narrow(int64_t num_tokens, int64_t rows, int32_t num_experts, bo
 // 256x256 kernel of GEMM 1 needs beyond the routing tables; mid() what comes between
 // the GEMMs.
 extern "C++" {
+// route_topk, expert_offsets and scatter of at most kSmallTok tokens in one launch.
+static int launch_route_small(const float* logits, const MoeWorkspace& w, int64_t num_tokens, int32_t num_experts,
+                              int32_t top_k, int narrow_max, int32_t* narrow_info, hipStream_t s) {
+  const int per_lane = (num_experts + 15) / 16;  // experts per lane of a token's 16-lane row
+  auto kern = per_lane <= 1 ? route_small_kernel<1> : per_lane <= 2 ? route_small_kernel<2>
+            : per_lane <= 4 ? route_small_kernel<4> : per_lane <= 8 ? route_small_kernel<8>
+            : per_lane <= 16 ? route_small_kernel<16> : per_lane <= 32 ? route_small_kernel<32>
+                             : route_small_kernel<64>;
+  hk_launch(kern, dim3(1), dim3(kScanThreads), 0, s, logits, static_cast<int>(num_tokens), num_experts, top_k,
+            w.topk_idx, w.topk_w, w.counts, w.offsets, w.mtile_offsets, w.mtile_list, kBM, w.amax, w.tile_ctr,
+            narrow_max, narrow_info, w.perm, w.inv_perm);
+  return check_launch("route_small_kernel");
+}
+
 template <typename Prep, typename G1, typename Mid, typename G2>
 int moe_enqueue(const float* logits, const MoeWorkspace& w, int64_t num_tokens, int32_t num_experts, int32_t top_k,
                 int32_t hidden, void* out, hipStream_t s, NarrowPlan& plan, Prep prep, G1 gemm1, Mid mid, G2 gemm2) {
@@ -1123,14 +1137,20 @@ int moe_enqueue(const float* logits, const MoeWorkspace& w, int64_t num_tokens, 
   const int cus = device_cus();
   TimedCall timed_call;
   t_role = HKMOE_TIMING_ROUTE;
-  HK_TRY(hkmoe_route_topk(logits, num_tokens, num_experts, top_k, w.topk_idx, w.topk_w, w.block_counts, s));
-  t_role = HKMOE_TIMING_OFFSETS;
-  HK_TRY(launch_expert_offsets(w.block_counts, num_tokens, num_experts, w.counts, w.offsets, w.block_base,
-                               w.mtile_offsets, w.mtile_list, w.amax, w.tile_ctr, plan.on() ? nc.max_rows : 0,
-                               plan.on() ? w.narrow_info : nullptr, s));
-  t_role = HKMOE_TIMING_SCATTER;
-  HK_TRY(hkmoe_scatter(w.topk_idx, num_tokens, num_experts, top_k, w.offsets, w.block_base, w.perm, w.inv_perm,
-                       nullptr, nullptr, hidden, HKMOE_SCALE_TENSOR, nullptr, nullptr, s));
+  // (a timed call takes the three steps apart, so that each has a time of its own)
+  if (num_tokens <= kSmallTok && !timed_call.on) {
+    HK_TRY(launch_route_small(logits, w, num_tokens, num_experts, top_k, plan.on() ? nc.max_rows : 0,
+                              plan.on() ? w.narrow_info : nullptr, s));
+  } else {
+    HK_TRY(hkmoe_route_topk(logits, num_tokens, num_experts, top_k, w.topk_idx, w.topk_w, w.block_counts, s));
+    t_role = HKMOE_TIMING_OFFSETS;
+    HK_TRY(launch_expert_offsets(w.block_counts, num_tokens, num_experts, w.counts, w.offsets, w.block_base,
+                                 w.mtile_offsets, w.mtile_list, w.amax, w.tile_ctr, plan.on() ? nc.max_rows : 0,
+                                 plan.on() ? w.narrow_info : nullptr, s));
+    t_role = HKMOE_TIMING_SCATTER;
+    HK_TRY(hkmoe_scatter(w.topk_idx, num_tokens, num_experts, top_k, w.offsets, w.block_base, w.perm, w.inv_perm,
+                         nullptr, nullptr, hidden, HKMOE_SCALE_TENSOR, nullptr, nullptr, s));
+  }
   if (plan.seq) {
     // each 256x256 GEMM keeps every CU and skips the narrow experts' tiles; each
     // narrow GEMM then runs its items on every CU.  A token's k experts are

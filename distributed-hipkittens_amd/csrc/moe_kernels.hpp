@@ -24,40 +24,101 @@ constexpr int kTileCounters = 16;  // HKMOE_TILE_COUNTERS
 constexpr int kNarrowCounters = 4;  // narrow kernel item counters (GEMM 1, GEMM 2), then their
                                     // active-slot counters
 
-__device__ __forceinline__ bool route_better(float av, int ai, float bv, int bi) {
-  if (bi < 0) return ai >= 0;
-  if (ai < 0) return false;
-  return av > bv || (av == bv && ai < bi);
+// Logit as an unsigned key of the same order; equal logits (-0 and +0 too) have
+// equal keys.  A NaN is below every number, and 0 is below every key.
+__device__ __forceinline__ uint32_t route_key(float v) {
+  const uint32_t u = __float_as_uint(v + 0.0f);  // -0 -> +0
+  const uint32_t k = u ^ (static_cast<uint32_t>(static_cast<int32_t>(u) >> 31) | 0x80000000u);
+  return __builtin_isnan(v) ? 1u : k;
+}
+__device__ __forceinline__ float route_value(uint32_t key) {
+  const uint32_t u = (key & 0x80000000u) ? key ^ 0x80000000u : ~key;
+  return __uint_as_float(key == 1u ? 0x7fc00000u : u);
 }
 
-// One level of a row argmax: every lane takes the better of its own entry and
-// the one that DPP control CTRL (a permutation within rows of 16 lanes) brings.
-template <int CTRL>
-__device__ __forceinline__ void route_best_dpp(float& bv, int& bi) {
-  const float ov =
-      __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(bv), __float_as_int(bv), CTRL, 0xf, 0xf, false));
-  const int oi = __builtin_amdgcn_update_dpp(bi, bi, CTRL, 0xf, 0xf, false);
-  if (route_better(ov, oi, bv, bi)) {
-    bv = ov;
-    bi = oi;
-  }
+// Reduction over the row of 16 lanes by DPP swaps (quad pairs, quad swap,
+// half-row and row mirrors); every lane gets the result.
+template <typename Op>
+__device__ __forceinline__ uint32_t row16_reduce(uint32_t v, Op op) {
+  auto step = [&](auto ctrl) __attribute__((always_inline)) {
+    v = op(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v),
+                                                                decltype(ctrl)::value, 0xf, 0xf, false)));
+  };
+  step(std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  step(std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  step(std::integral_constant<int, 0x141>{});  // row_half_mirror
+  step(std::integral_constant<int, 0x140>{});  // row_mirror
+  return v;
 }
 
 // ---------------------------------------------------------------------------
 // 1. top-k + softmax + per-block histogram.  16 lanes (one row of the wave) per
 //    token, 4 tokens per wave; lane s of a token's row holds experts c*16 + s,
 //    c < CH (CH: power of two >= ceil(E / 16)).  Each of the k rounds takes
-//    the lane's best untaken expert and reduces the row by DPP swaps (quad
-//    pairs, quad swap, half-row and row mirrors): VALU only, and a round's
-//    work is shared by four tokens.  route_better is a total order, so the
-//    reduction order does not change the winner.
+//    the row's largest key (integer maxima, then DPP swaps), the lowest expert
+//    that has it (integer minima), and clears that key: VALU only, and a round's work
+//    is shared by four tokens.  Carrying (value, expert) pairs through every
+//    comparison took about twice the instructions.
 // ---------------------------------------------------------------------------
+// Token t's top-k on its row of 16 lanes: writes topk_idx / topk_w; lane sub gets
+// the experts of slots sub and sub + 16 (where < top_k).
+struct TopkLane {
+  int e0, e1;
+};
+template <int CH>
+__device__ __forceinline__ TopkLane route_token(const float* __restrict__ logits, int t, int num_experts, int top_k,
+                                                int32_t* __restrict__ topk_idx, float* __restrict__ topk_w) {
+  const int sub = threadIdx.x & 15;
+  const float* row = logits + static_cast<int64_t>(t) * num_experts;
+  uint32_t key[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int id = c * 16 + sub;
+    key[c] = (id < num_experts) ? route_key(row[id]) : 0u;
+  }
+  uint32_t first = 0, mk0 = 1, mk1 = 1;  // winners j (lane j % 16): j < 16 in mk0 / mi0, else mk1 / mi1
+  int mi0 = 0, mi1 = 0;
+  for (int j = 0; j < top_k; ++j) {
+    uint32_t m = key[0];
+#pragma unroll
+    for (int c = 1; c < CH; ++c) m = max(m, key[c]);
+    m = row16_reduce(m, [](uint32_t x, uint32_t y) { return max(x, y); });
+    uint32_t best = 0xffffffffu;
+#pragma unroll
+    for (int c = CH - 1; c >= 0; --c) best = (key[c] == m) ? static_cast<uint32_t>(c * 16) : best;
+    best = best == 0xffffffffu ? best : best + sub;
+    best = row16_reduce(best, [](uint32_t x, uint32_t y) { return min(x, y); });
+    const int mine = static_cast<int>(best) - sub;  // 16c in the lane that holds the winner
+#pragma unroll
+    for (int c = 0; c < CH; ++c) key[c] = (mine == c * 16) ? 0u : key[c];
+    if (j == 0) first = m;
+    if ((j & 15) == sub) {
+      if (j < 16) { mk0 = m; mi0 = static_cast<int>(best); } else { mk1 = m; mi1 = static_cast<int>(best); }
+    }
+  }
+  const float v0 = route_value(first), mv0 = route_value(mk0), mv1 = route_value(mk1);
+  // softmax over the winners: exp(v_j - v_0) / sum_j exp(v_j - v_0), the sum
+  // taken in j order
+  const float ex0 = (sub < top_k) ? expf(mv0 - v0) : 0.0f;
+  const float ex1 = (sub + 16 < top_k) ? expf(mv1 - v0) : 0.0f;
+  float tot = 0.0f;
+  for (int j = 0; j < top_k; ++j) tot = tot + __shfl(j < 16 ? ex0 : ex1, j & 15, 16);
+  if (sub < top_k) {
+    topk_idx[static_cast<int64_t>(t) * top_k + sub] = mi0;
+    topk_w[static_cast<int64_t>(t) * top_k + sub] = ex0 / tot;
+  }
+  if (sub + 16 < top_k) {
+    topk_idx[static_cast<int64_t>(t) * top_k + sub + 16] = mi1;
+    topk_w[static_cast<int64_t>(t) * top_k + sub + 16] = ex1 / tot;
+  }
+  return TopkLane{mi0, mi1};
+}
+
 template <int CH>
 __global__ __launch_bounds__(kTopkThreads) void route_topk_kernel(
     const float* __restrict__ logits, int num_tokens, int num_experts, int top_k,
     int32_t* __restrict__ topk_idx, float* __restrict__ topk_w, int32_t* __restrict__ block_counts) {
   static_assert(kTopkThreads == 16 * kRouteTok, "one 16-lane row per token");
-  static_assert(CH <= 64, "taken mask");
   __shared__ int hist[kMaxExperts];
   const int sub = threadIdx.x & 15;
   for (int e = threadIdx.x; e < num_experts; e += kTopkThreads) hist[e] = 0;
@@ -65,53 +126,9 @@ __global__ __launch_bounds__(kTopkThreads) void route_topk_kernel(
 
   const int t = blockIdx.x * kRouteTok + (threadIdx.x >> 4);
   if (t < num_tokens) {  // uniform over the token's row
-    const float* row = logits + static_cast<int64_t>(t) * num_experts;
-    float v[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int id = c * 16 + sub;
-      v[c] = (id < num_experts) ? row[id] : 0.0f;
-    }
-    uint64_t taken = 0;
-    float v0 = 0.0f, mv0 = 0.0f, mv1 = 0.0f;  // winners j (lane j % 16): j < 16 in mv0, else mv1
-    int mi0 = 0, mi1 = 0;
-    for (int j = 0; j < top_k; ++j) {
-      float bv = 0.0f;
-      int bi = -1;
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const int id = c * 16 + sub;
-        if (id < num_experts && !((taken >> c) & 1u) && route_better(v[c], id, bv, bi)) {
-          bv = v[c];
-          bi = id;
-        }
-      }
-      route_best_dpp<0xB1>(bv, bi);   // quad_perm [1,0,3,2]
-      route_best_dpp<0x4E>(bv, bi);   // quad_perm [2,3,0,1]
-      route_best_dpp<0x141>(bv, bi);  // row_half_mirror
-      route_best_dpp<0x140>(bv, bi);  // row_mirror
-      if ((bi & 15) == sub) taken |= uint64_t{1} << (bi >> 4);
-      if (j == 0) v0 = bv;
-      if ((j & 15) == sub) {
-        if (j < 16) { mv0 = bv; mi0 = bi; } else { mv1 = bv; mi1 = bi; }
-      }
-    }
-    // softmax over the winners: exp(v_j - v_0) / sum_j exp(v_j - v_0), the sum
-    // taken in j order
-    const float ex0 = (sub < top_k) ? expf(mv0 - v0) : 0.0f;
-    const float ex1 = (sub + 16 < top_k) ? expf(mv1 - v0) : 0.0f;
-    float tot = 0.0f;
-    for (int j = 0; j < top_k; ++j) tot = tot + __shfl(j < 16 ? ex0 : ex1, j & 15, 16);
-    if (sub < top_k) {
-      topk_idx[static_cast<int64_t>(t) * top_k + sub] = mi0;
-      topk_w[static_cast<int64_t>(t) * top_k + sub] = ex0 / tot;
-      atomicAdd(&hist[mi0], 1);
-    }
-    if (sub + 16 < top_k) {
-      topk_idx[static_cast<int64_t>(t) * top_k + sub + 16] = mi1;
-      topk_w[static_cast<int64_t>(t) * top_k + sub + 16] = ex1 / tot;
-      atomicAdd(&hist[mi1], 1);
-    }
+    const TopkLane r = route_token<CH>(logits, t, num_experts, top_k, topk_idx, topk_w);
+    if (sub < top_k) atomicAdd(&hist[r.e0], 1);
+    if (sub + 16 < top_k) atomicAdd(&hist[r.e1], 1);
   }
   __syncthreads();
   for (int e = threadIdx.x; e < num_experts; e += kTopkThreads)
@@ -239,13 +256,79 @@ __device__ __forceinline__ void block_exclusive_scan_n(int (&v)[N], int (*wave_t
   for (int i = 0; i < N; ++i) v[i] = wave_tot[wave][i] + incl[i] - v[i];
 }
 
+// The tables that follow from the experts' row counts (thread = expert, cnt 0
+// past num_experts): offsets, M-tile offsets and list, counters reset.  Returns the
+// expert's first row.
+struct OffsetsLds {
+  int wave_tot[kScanThreads / 64][5];
+  int n_head, n_tail;
+};
+__device__ __forceinline__ int expert_offsets_tables(int e, int cnt, OffsetsLds& lds, int num_experts,
+                                                     int32_t* __restrict__ offsets,
+                                                     int32_t* __restrict__ mtile_offsets,
+                                                     int32_t* __restrict__ mtile_list, int tile_m, float* amax_reset,
+                                                     int32_t* tile_counters, int narrow_max, int32_t* narrow_info) {
+  const int mt = (cnt + tile_m - 1) / tile_m;
+  // M-tile list [(expert, first row)]: first the experts with at least one
+  // full tile, each with all its tiles (full ones, then its partial one), in
+  // expert order; then the single partial tiles of the smaller experts; last,
+  // with narrow_max > 0, the experts of 1..narrow_max rows, which the narrow
+  // kernel takes (their count goes to narrow_info[0]).  Tiles of nearly equal
+  // cost sit together in the grouped GEMMs' schedule, so the workgroups that
+  // share a tile block stay in step and reuse its operands in L2, and a large
+  // expert's partial tile runs while its weights are still in L2 / MALL
+  // instead of streaming them once more.
+  const int q_full = cnt / tile_m;
+  const int q_part = (cnt % tile_m) ? 1 : 0;
+  const int q_head = q_full > 0 ? q_full + q_part : 0;
+  const int q_narrow = (q_full == 0 && cnt > 0 && cnt <= narrow_max) ? 1 : 0;
+  const int q_tail = (q_full > 0 || q_narrow) ? 0 : q_part;
+  // one pass of exclusive scans over the experts: row offsets, M-tile
+  // offsets, and the list positions of the three kinds of tiles
+  int sc[5] = {cnt, mt, q_head, q_tail, q_narrow};
+  block_exclusive_scan_n<5>(sc, lds.wave_tot);
+  const int off = sc[0], moff = sc[1], head_base = sc[2], tail_base = sc[3], narrow_base = sc[4];
+  if (e < num_experts) {
+    offsets[e] = off;
+    mtile_offsets[e] = moff;
+  }
+  if (e == num_experts - 1) {
+    offsets[num_experts] = off + cnt;
+    mtile_offsets[num_experts] = moff + mt;
+    lds.n_head = head_base + q_head;
+    lds.n_tail = tail_base + q_tail;
+    if (mtile_list != nullptr && narrow_info != nullptr) narrow_info[0] = narrow_base + q_narrow;
+  }
+  if (mtile_list != nullptr) {
+    __syncthreads();
+    if (e < num_experts) {
+      for (int s = 0; s < q_head; ++s) {
+        mtile_list[2 * (head_base + s)] = e;
+        mtile_list[2 * (head_base + s) + 1] = off + s * tile_m;
+      }
+      if (q_tail) {
+        mtile_list[2 * (lds.n_head + tail_base)] = e;
+        mtile_list[2 * (lds.n_head + tail_base) + 1] = off;
+      }
+      if (q_narrow) {
+        mtile_list[2 * (lds.n_head + lds.n_tail + narrow_base)] = e;
+        mtile_list[2 * (lds.n_head + lds.n_tail + narrow_base) + 1] = off;
+      }
+    }
+  }
+  const int tid = threadIdx.x;
+  if (narrow_info != nullptr && tid >= 1 && tid < 1 + kNarrowCounters) narrow_info[tid] = 0;
+  if (tid == 0 && amax_reset != nullptr) *amax_reset = 0.0f;
+  if (tile_counters != nullptr && tid < kTileCounters) tile_counters[tid] = 0;
+  return off;
+}
+
 __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
     int num_experts, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
     int32_t* __restrict__ mtile_offsets, int32_t* __restrict__ mtile_list, int tile_m,
     float* amax_reset, int32_t* tile_counters, int narrow_max, int32_t* narrow_info,
     const int32_t* __restrict__ block_counts, int fused_nblk, int32_t* __restrict__ block_base) {
-  __shared__ int wave_tot[kScanThreads / 64][5];
-  __shared__ int n_head, n_tail;
+  __shared__ OffsetsLds lds;
   const int e = threadIdx.x;  // E <= kScanThreads
   int cnt = 0;
   if (fused_nblk >= 0) {
@@ -266,58 +349,55 @@ __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
   } else if (e < num_experts) {
     cnt = counts[e];
   }
-  const int mt = (cnt + tile_m - 1) / tile_m;
-  // M-tile list [(expert, first row)]: first the experts with at least one
-  // full tile, each with all its tiles (full ones, then its partial one), in
-  // expert order; then the single partial tiles of the smaller experts; last,
-  // with narrow_max > 0, the experts of 1..narrow_max rows, which the narrow
-  // kernel takes (their count goes to narrow_info[0]).  Tiles of nearly equal
-  // cost sit together in the grouped GEMMs' schedule, so the workgroups that
-  // share a tile block stay in step and reuse its operands in L2, and a large
-  // expert's partial tile runs while its weights are still in L2 / MALL
-  // instead of streaming them once more.
-  const int q_full = cnt / tile_m;
-  const int q_part = (cnt % tile_m) ? 1 : 0;
-  const int q_head = q_full > 0 ? q_full + q_part : 0;
-  const int q_narrow = (q_full == 0 && cnt > 0 && cnt <= narrow_max) ? 1 : 0;
-  const int q_tail = (q_full > 0 || q_narrow) ? 0 : q_part;
-  // one pass of exclusive scans over the experts: row offsets, M-tile
-  // offsets, and the list positions of the three kinds of tiles
-  int sc[5] = {cnt, mt, q_head, q_tail, q_narrow};
-  block_exclusive_scan_n<5>(sc, wave_tot);
-  const int off = sc[0], moff = sc[1], head_base = sc[2], tail_base = sc[3], narrow_base = sc[4];
-  if (e < num_experts) {
-    offsets[e] = off;
-    mtile_offsets[e] = moff;
+  expert_offsets_tables(e, cnt, lds, num_experts, offsets, mtile_offsets, mtile_list, tile_m, amax_reset,
+                        tile_counters, narrow_max, narrow_info);
+}
+
+// Routing of at most kSmallTok tokens in one launch: top-k (16 lanes per token, as
+// route_topk_kernel), offsets and the stable permutation.  Each expert keeps
+// the set of its tokens as a 64-bit mask in LDS (a token names an expert at most once),
+// so its count is a population count and a slot's place among the expert's rows
+// the count of the mask below its token.  Three launches and their latencies in a
+// decode step's critical path become one: E=128, k=8: 14.5 -> 8.1 us at T=1 (plus two
+// launch gaps), 21.8 -> 12.7 us at T=64.
+constexpr int kSmallTok = 64;
+template <int CH>
+__global__ __launch_bounds__(kScanThreads) void route_small_kernel(
+    const float* __restrict__ logits, int num_tokens, int num_experts, int top_k, int32_t* __restrict__ topk_idx,
+    float* __restrict__ topk_w, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ mtile_offsets, int32_t* __restrict__ mtile_list, int tile_m, float* amax_reset,
+    int32_t* tile_counters, int narrow_max, int32_t* narrow_info, int32_t* __restrict__ perm,
+    int32_t* __restrict__ inv_perm) {
+  static_assert(kScanThreads == 16 * kSmallTok && kScanThreads >= kMaxExperts, "thread = token lane, then expert");
+  __shared__ OffsetsLds lds;
+  __shared__ uint32_t tokens[kMaxExperts][2];  // bit t of the expert's token set
+  __shared__ int first[kMaxExperts];
+  const int tid = threadIdx.x, sub = tid & 15, t = tid >> 4;
+  tokens[tid][0] = tokens[tid][1] = 0;
+  __syncthreads();
+  TopkLane r{0, 0};
+  if (t < num_tokens) {  // uniform over the token's row
+    r = route_token<CH>(logits, t, num_experts, top_k, topk_idx, topk_w);
+    if (sub < top_k) atomicOr(&tokens[r.e0][t >> 5], 1u << (t & 31));
+    if (sub + 16 < top_k) atomicOr(&tokens[r.e1][t >> 5], 1u << (t & 31));
   }
-  if (e == num_experts - 1) {
-    offsets[num_experts] = off + cnt;
-    mtile_offsets[num_experts] = moff + mt;
-    n_head = head_base + q_head;
-    n_tail = tail_base + q_tail;
-    if (mtile_list != nullptr && narrow_info != nullptr) narrow_info[0] = narrow_base + q_narrow;
+  __syncthreads();
+  const int cnt = tid < num_experts ? __popc(tokens[tid][0]) + __popc(tokens[tid][1]) : 0;
+  if (tid < num_experts) counts[tid] = cnt;
+  first[tid] = expert_offsets_tables(tid, cnt, lds, num_experts, offsets, mtile_offsets, mtile_list, tile_m, amax_reset,
+                                     tile_counters, narrow_max, narrow_info);
+  __syncthreads();
+  if (t < num_tokens) {
+    auto place = [&](int e, int j) {
+      const uint64_t set = tokens[e][0] | (static_cast<uint64_t>(tokens[e][1]) << 32);
+      const int p = first[e] + __popcll(set & ((uint64_t{1} << t) - 1));
+      const int f = t * top_k + j;
+      perm[p] = f;
+      inv_perm[f] = p;
+    };
+    if (sub < top_k) place(r.e0, sub);
+    if (sub + 16 < top_k) place(r.e1, sub + 16);
   }
-  if (mtile_list != nullptr) {
-    __syncthreads();
-    if (e < num_experts) {
-      for (int s = 0; s < q_head; ++s) {
-        mtile_list[2 * (head_base + s)] = e;
-        mtile_list[2 * (head_base + s) + 1] = off + s * tile_m;
-      }
-      if (q_tail) {
-        mtile_list[2 * (n_head + tail_base)] = e;
-        mtile_list[2 * (n_head + tail_base) + 1] = off;
-      }
-      if (q_narrow) {
-        mtile_list[2 * (n_head + n_tail + narrow_base)] = e;
-        mtile_list[2 * (n_head + n_tail + narrow_base) + 1] = off;
-      }
-    }
-  }
-  const int tid = threadIdx.x;
-  if (narrow_info != nullptr && tid >= 1 && tid < 1 + kNarrowCounters) narrow_info[tid] = 0;
-  if (tid == 0 && amax_reset != nullptr) *amax_reset = 0.0f;
-  if (tile_counters != nullptr && tid < kTileCounters) tile_counters[tid] = 0;
 }
 
 // ---------------------------------------------------------------------------

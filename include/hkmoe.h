@@ -322,7 +322,9 @@ int hkmoe_get_narrow(int32_t* cus, int32_t* max_rows, int32_t* wide_share);
  *     hkmoe_moe_forward / hkmoe_moe_forward_mx / hkmoe_moe_forward_noalloc calls on
  *     the current device, cycling over `calls` sets of events (call i uses set
  *     i % calls, counting from this call); 0 turns it off.  Creates (and
- *     frees) events: not for use under graph capture.
+ *     frees) events: not for use under graph capture.  A timed call of at most
+ *     64 tokens routes in three kernels (ROUTE, OFFSETS, SCATTER), where an
+ *     untimed one uses a single kernel; every other launch is the same.
  *   hkmoe_kernel_timing_read(set, begin_ms, end_ms, n): after the timed calls
  *     completed (the caller synchronises), the start and end of each role's
  *     kernel in ms from the start of the call's first kernel, or -1 for both
