@@ -565,7 +565,7 @@ struct AuxJoin {
 int launch_expert_offsets(const int32_t* block_counts, int64_t num_tokens, int32_t num_experts,
                           int32_t* counts, int32_t* offsets, int32_t* block_base,
                           int32_t* mtile_offsets, int32_t* mtile_list, float* amax_reset,
-                          int32_t* tile_counters, int narrow_max, int32_t* narrow_info,
+                          int32_t* tile_counters, int narrow_max, int narrow_min, int32_t* narrow_info,
                           hipStream_t stream) {
   const int nblk = route_blocks(num_tokens);
   // few routing blocks: expert_offsets_kernel also does the block scan (one
@@ -580,7 +580,7 @@ int launch_expert_offsets(const int32_t* block_counts, int64_t num_tokens, int32
     if (timed) t_role = HKMOE_TIMING_OFFSETS;
   }
   hk_launch(expert_offsets_kernel, dim3(1), dim3(kScanThreads), 0, stream, num_experts, counts, offsets,
-            mtile_offsets, mtile_list, kBM, amax_reset, tile_counters, narrow_max, narrow_info,
+            mtile_offsets, mtile_list, kBM, amax_reset, tile_counters, narrow_max, narrow_min, narrow_info,
             block_counts, fuse ? nblk : -1, block_base);
   return check_launch("expert_offsets_kernel");
 }
@@ -670,7 +670,7 @@ int hkmoe_expert_offsets(const int32_t* block_counts, int64_t num_tokens, int32_
   HK_REQUIRE(num_tokens >= 0, "expert_offsets: bad T");
   HK_REQUIRE(num_tokens == 0 || block_counts, "expert_offsets: null block_counts");
   return launch_expert_offsets(block_counts, num_tokens, num_experts, counts, offsets, block_base,
-                               mtile_offsets, mtile_list, amax_reset, tile_counters, 0, nullptr,
+                               mtile_offsets, mtile_list, amax_reset, tile_counters, 0, 0, nullptr,
                                static_cast<hipStream_t>(stream));
 }
 
@@ -688,7 +688,7 @@ int hkmoe_expert_offsets_narrow(const int32_t* block_counts, int64_t num_tokens,
   HK_REQUIRE(narrow_max >= 0 && narrow_max <= kNarrowRows, "expert_offsets_narrow: narrow_max=%d outside [0, %d]",
              narrow_max, kNarrowRows);
   return launch_expert_offsets(block_counts, num_tokens, num_experts, counts, offsets, block_base,
-                               mtile_offsets, mtile_list, amax_reset, tile_counters, narrow_max, narrow_info,
+                               mtile_offsets, mtile_list, amax_reset, tile_counters, narrow_max, 0, narrow_info,
                                static_cast<hipStream_t>(stream));
 }
 
@@ -1080,6 +1080,7 @@ size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t
 struct NarrowPlan {
   NarrowConfig cfg{};
   bool seq = false;
+  int min_experts = 0;  // with fewer small experts the 256x256 kernels take them all
   AuxStreams* aux = nullptr;
   std::unique_lock<std::mutex> lock;  // held while the fork / join is enqueued
   bool on() const { return seq || aux != nullptr; }
@@ -1089,23 +1090,46 @@ struct NarrowPlan {
 // the 256x256 kernels alone).  tuned: block scales and at most 64 K steps, an even
 // number, in both GEMMs; the lines above were measured there.  For the rest
 // (per-tensor and MX scales, other step counts) the 256x256 kernels lose less to
-// small experts, and two narrow launches that find none cost 8 us: they
-// take the narrow path
+// small experts, and with experts of both kinds each kernel's start and tail cost
+// 30 us or so.  They take the narrow path
 //   with at most max_rows tokens (every expert is narrow): E=8 H=4096 I=14336
-//     per-tensor T=29 328 -> 246 us, E=128 H=4096 I=1536 MX T=48 454 -> 368 us;
-//   and from 256 experts on, where skewed routing leaves many small ones beside a few
-//     large: H=7168 I=2048 per-tensor T=1700 1397 -> 1309 us, MX T=3001 1865 -> 1802 us,
-//     T=8192 3631 -> 3312 us (uniform routing, no small expert: 2211 / 2216 us).  With
-//     fewer experts the two kernels one after the other lose what the smaller one
-//     gains: E=8 per-tensor T=200 skewed 350 / 411 us, E=128 MX T=600 429 / 469 us.
-static int plan_narrow(int64_t num_tokens, int64_t rows, int32_t num_experts, bool tuned, bool aux_ok, hipStream_t s,
-                       NarrowPlan* plan) {
+//     per-tensor T=29 326 -> 245 us, E=128 H=4096 I=1536 MX T=48 453 -> 358 us.
+//     Row-major weights, which the narrow kernel reads at 5.0-5.4 TB/s, only up to
+//     kRowMajorBytes of them (T=64 above: 498 -> 482 us; the 256x256 kernels reach
+//     5.9 on more: E=256 H=7168 I=2048 T=40 1376, narrow 1505 us);
+//   and packed ones from 256 experts on, where skewed routing leaves many small
+//     experts beside a few large: if at least kMixedExperts of them are small (the
+//     device decides; uniform T=2500, 15 small experts, lost 2%, skewed T=70, one
+//     expert above 64 rows beside 50, 5%).  H=7168 I=2048, skewed, per-tensor T=2000 /
+//     4000 / 8192 1484 / 2195 / 3488 -> 1435 / 2115 / 3404 us, uniform T=700 1959 ->
+//     1718.  MX on one stream up to kMixedSeqRows rows per expert (T=5000 2580 -> 2482
+//     us, on two 2654), on two above (T=6500 3175 -> 2786, on one 3034).  With fewer
+//     experts the two kernels one after the other lose what the smaller one gains: E=8
+//     per-tensor T=200 skewed 350 / 411 us, E=128 MX T=600 429 / 469 us.
+constexpr int kMixedExperts = 112;
+constexpr int64_t kMixedSeqRows = 176, kMixedTensorRows = 256;
+constexpr int64_t kRowMajorBytes = 2500000000;
+struct NarrowCall {
+  int64_t tokens, rows;
+  int32_t experts;
+  int64_t expert_bytes;  // both weights of one expert
+  bool tuned, tensor, packed, aux_ok;
+};
+static int plan_narrow(const NarrowCall& c, hipStream_t s, NarrowPlan* plan) {
   plan->cfg = narrow_config();
   const int64_t max_rows = plan->cfg.max_rows;
   if (plan->cfg.cus <= 0 || max_rows <= 0) return HKMOE_OK;
-  if (!tuned && num_tokens > max_rows && num_experts < 256) return HKMOE_OK;
-  plan->seq = num_tokens <= max_rows || rows <= 2 * num_experts * max_rows;
-  if (plan->seq || !aux_ok) return HKMOE_OK;
+  if (c.tuned) {
+    plan->seq = c.tokens <= max_rows || c.rows <= 2 * c.experts * max_rows;
+  } else if (c.tokens <= max_rows) {
+    plan->seq = c.packed || std::min<int64_t>(c.rows, c.experts) * c.expert_bytes <= kRowMajorBytes;
+    if (!plan->seq) return HKMOE_OK;
+  } else {
+    if (c.experts < 256 || !c.packed) return HKMOE_OK;
+    plan->min_experts = kMixedExperts;
+    plan->seq = c.rows <= c.experts * (c.tensor ? kMixedTensorRows : kMixedSeqRows);
+  }
+  if (plan->seq || !c.aux_ok) return HKMOE_OK;
   HK_TRY(get_aux(s, &plan->aux));
   if (plan->aux) plan->lock = std::unique_lock<std::mutex>(g_aux_mu);
   return HKMOE_OK;
@@ -1146,7 +1170,7 @@ int moe_enqueue(const float* logits, const MoeWorkspace& w, int64_t num_tokens, 
     t_role = HKMOE_TIMING_OFFSETS;
     HK_TRY(launch_expert_offsets(w.block_counts, num_tokens, num_experts, w.counts, w.offsets, w.block_base,
                                  w.mtile_offsets, w.mtile_list, w.amax, w.tile_ctr, plan.on() ? nc.max_rows : 0,
-                                 plan.on() ? w.narrow_info : nullptr, s));
+                                 plan.min_experts, plan.on() ? w.narrow_info : nullptr, s));
     t_role = HKMOE_TIMING_SCATTER;
     HK_TRY(hkmoe_scatter(w.topk_idx, num_tokens, num_experts, top_k, w.offsets, w.block_base, w.perm, w.inv_perm,
                          nullptr, nullptr, hidden, HKMOE_SCALE_TENSOR, nullptr, nullptr, s));
@@ -1268,7 +1292,8 @@ static int moe_forward_impl(const void* x_q, const float* x_scale, const float* 
   auto s = static_cast<hipStream_t>(stream);
   NarrowPlan plan;
   const bool tuned = block && narrow_part_steps(hidden / kBK) && narrow_part_steps(inter / kBK);
-  HK_TRY(plan_narrow(num_tokens, rows, num_experts, tuned, aux_ok && block, s, &plan));
+  HK_TRY(plan_narrow({num_tokens, rows, num_experts, 3ll * inter * hidden, tuned, !block,
+                      w_layout == HKMOE_W_PACKED, aux_ok && block}, s, &plan));
   return moe_enqueue(
       logits, w, num_tokens, num_experts, top_k, hidden, out, s, plan, [] { return HKMOE_OK; },
       // GEMM 1 reads token rows through perm; with block scales it writes the
@@ -1625,7 +1650,8 @@ int hkmoe_moe_forward_mx(const void* x_q, const void* x_e8m0, const float* logit
   const int64_t rows = num_tokens * top_k;
   auto s = static_cast<hipStream_t>(stream);
   NarrowPlan plan;
-  HK_TRY(plan_narrow(num_tokens, rows, num_experts, false, true, s, &plan));
+  HK_TRY(plan_narrow({num_tokens, rows, num_experts, 3ll * inter * hidden, false, false,
+                      w_layout == HKMOE_W_PACKED, true}, s, &plan));
   return moe_enqueue(
       logits, w, num_tokens, num_experts, top_k, hidden, out, s, plan,
       // token exponents -> tile-aligned words in expert order (x rows stay in place)

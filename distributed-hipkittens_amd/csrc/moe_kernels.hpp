@@ -326,7 +326,7 @@ __device__ __forceinline__ int expert_offsets_tables(int e, int cnt, OffsetsLds&
 __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
     int num_experts, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
     int32_t* __restrict__ mtile_offsets, int32_t* __restrict__ mtile_list, int tile_m,
-    float* amax_reset, int32_t* tile_counters, int narrow_max, int32_t* narrow_info,
+    float* amax_reset, int32_t* tile_counters, int narrow_max, int narrow_min, int32_t* narrow_info,
     const int32_t* __restrict__ block_counts, int fused_nblk, int32_t* __restrict__ block_base) {
   __shared__ OffsetsLds lds;
   const int e = threadIdx.x;  // E <= kScanThreads
@@ -349,6 +349,8 @@ __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
   } else if (e < num_experts) {
     cnt = counts[e];
   }
+  // fewer than narrow_min experts for the narrow kernel: none
+  if (narrow_min > 0 && __syncthreads_count(cnt > 0 && cnt <= narrow_max) < narrow_min) narrow_max = 0;
   expert_offsets_tables(e, cnt, lds, num_experts, offsets, mtile_offsets, mtile_list, tile_m, amax_reset,
                         tile_counters, narrow_max, narrow_info);
 }

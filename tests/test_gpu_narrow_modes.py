@@ -43,7 +43,8 @@ def _layer(hk, mode, H, I, E, k, packed, gen):
 def _inputs(hk, mode, T, H, E, gen):
     x = torch.randn(T, H, device="cuda", generator=gen)
     logits = torch.randn(T, E, device="cuda", generator=gen)
-    logits -= 1.1 * torch.log(torch.arange(1, E + 1, device="cuda").float())  # skewed routing
+    skew = 0.55 if E == 256 else 1.1
+    logits -= skew * torch.log(torch.arange(1, E + 1, device="cuda").float())
     return {"block": hk.quant_group, "mx": hk.quant_mx, "tensor": hk.quant_tensor}[mode](x) + (logits,)
 
 
@@ -54,7 +55,10 @@ def test_narrow_matches_wide(hk, narrow_restore, mode, shape, packed):
     H, I, E, k = shape
     gen = torch.Generator(device="cuda").manual_seed(H + I + E)
     layer = _layer(hk, mode, H, I, E, k, packed, gen)
-    for T in (1, 3, 16, 17, 64, 65, 150, 400):
+    # with 256 experts and weights in the packed layout, 65 tokens leave fewer small
+    # experts than the mixed schedules ask for, 400 take them one after the other and
+    # 11400 (178 rows per expert) MX and block scales on two streams
+    for T in (1, 3, 16, 17, 64, 65, 150, 400) + ((11400,) if E == 256 else ()):
         args = _inputs(hk, mode, T, H, E, gen)
         hk.tk_kernel.set_narrow(0, 64, 0)
         off = layer(*args).clone()
@@ -64,9 +68,9 @@ def test_narrow_matches_wide(hk, narrow_restore, mode, shape, packed):
             torch.cuda.synchronize()
             assert torch.equal(on.view(torch.int16), off.view(torch.int16)), (T, setting)
         assert bool(torch.isfinite(off.float()).all())
-    if E == 256:  # 400 tokens: experts of both kinds
-        counts = torch.bincount(torch.topk(args[-1], k).indices.flatten(), minlength=E)
-        assert bool((counts > 64).any()) and bool(((counts > 0) & (counts <= 16)).any())
+        if E == 256 and T >= 400:  # experts of both kinds, enough small ones
+            counts = torch.bincount(torch.topk(args[-1], k).indices.flatten(), minlength=E)
+            assert bool((counts > 64).any()) and int(((counts > 0) & (counts <= 64)).sum()) >= 112
 
 
 def test_mx_unaligned_exponents(hk):
