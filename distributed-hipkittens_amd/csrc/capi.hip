@@ -227,15 +227,14 @@ int launch_gemm_skinny(SkinnyParams p, bool f32out, hipStream_t stream) {
 // rounds of workgroups over the CUs x (ramp + K steps x time per step), or B's
 // stream from HBM where that is longer (a tenth of the compute term breaks ties
 // there).  The constants are fits to graph-replayed launches with three operand
-// copies; on 256 other shapes (M = 1 .. 10000, N = 512 .. 7168, K = 512 .. 14336,
-// both outputs and modes) the pick costs 0.4% over the best kernel on average,
-// 21% at worst.
-//   split-K strips against 128x128 tiles: 17x8192x2048 5.2 / 11.0 us, 64x2048x8192
-//     7.5 / 33, 256x4096x4096 11.6 / 19, 1024x1024x4096 11.6 / 19 (and losing:
-//     1024x4096x4096 40 / 22)
-//   128x128 against 256x256 tiles: 2048^3 14.5 / 25.6 us, 2048x4096x4096 43 / 48,
-//     4096^3 84 / 52, 2048x7168x2048 46 / 30
-// MX: the scaled MFMA's steps take longer in every kernel, most in the 128x128 one.
+// copies; on 90 other shapes (M = 24 .. 3333, N = 1024 .. 7168, K = 1536 .. 14336,
+// both outputs and modes) the pick costs 1.6% over the best kernel on average,
+// 11% at worst.
+//   split-K strips against 128x128 tiles: 128x2048x8192 9.3 / 29.5 us, 128x8192x1024
+//     6.4 / 7.0, 512x2048x2048 8.2 / 10.4 (and losing: 512x4096x4096 20.8 / 17.3)
+//   128x128 against 256x256 tiles: 2048^3 13.9 / 25.6 us, 2048x4096x4096 40.8 / 48.1
+//     (MX 44.8 / 52.5), 4096^3 79 / 51, 2048x8192x1024 28.3 / 21.2
+// MX: the scaled MFMA's steps take longer in every kernel.
 enum class DenseKernel { kStrip11, kStrip21, kStrip12, kStrip22, kStrip24, kStrip44, kTile128, kTile256 };
 
 // Tile blocks of the dense 256x256 kernel: 2^b M tiles x 32 / 2^b N tiles, one
@@ -274,7 +273,7 @@ DenseKernel pick_dense(int64_t m, int64_t n, int64_t k, bool f32out, bool mx) {
   {
     const uint64_t tiles = ((um + kSmTile - 1) / kSmTile) * (un / kSmTile);
     const double full = static_cast<double>(tiles / ncu), part = static_cast<double>(tiles % ncu);
-    const double busy = mx ? 0.74 : 0.58, idle = mx ? 0.68 : 0.47;  // per step, chip full / half full
+    const double busy = mx ? 0.58 : 0.52, idle = mx ? 0.51 : 0.40;  // per step, chip full / half full
     const double ramp = f32out ? 4.8 : 2.3;
     offer(DenseKernel::kTile128,
           2 + full * (ramp + ks * busy) + (part > 0 ? ramp + ks * (part <= cus / 2 ? idle : busy) : 0), 3 + nk / 2.0e6);

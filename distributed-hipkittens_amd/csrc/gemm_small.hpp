@@ -2,15 +2,19 @@
 // too many rows for the strips of gemm_skinny.hpp): C[M,N] = (sa*sb) * A[M,K] .
 // B[N,K]^T with per-tensor scales or MX exponents, bf16 or fp32 C.
 //
-// 128x128 output tiles, one non-persistent workgroup of 4 waves per tile, one
-// wave per SIMD, each wave 64x64 outputs: 4x4 v_mfma_f32_16x16x128_f8f6f4 per
-// K step, or (M32) 2x2 blocks of 32x32 outputs, each two
+// 128x128 output tiles, one non-persistent workgroup of 8 waves per tile, two
+// waves per SIMD, each wave 64x32 outputs: 4x2 v_mfma_f32_16x16x128_f8f6f4 per
+// K step, or (M32) two blocks of 32x32 outputs, each two
 // v_mfma_f32_32x32x64_f8f6f4 (the two 64-byte halves of the K step).
-// With one wave per SIMD there is no ping-pong partner: the wave overlaps its
-// own LDS fragment reads of step kt+1 with its MFMAs of step kt (two register
-// sets of fragments), and a 4-deep LDS ring fed by buffer->LDS DMA keeps three
-// K steps (96 KiB per CU) in flight (a fifth stage measured slower).  The 2048^3 GEMM (config 1) is 256 such
-// tiles, one per CU, where the 256x256 kernel has 64.
+// A K step is bounded by one wave's issue of fragment reads and DMA beside its
+// MFMAs: each wave overlaps its own LDS fragment reads of step kt+1 with its MFMAs
+// of step kt (two register sets of fragments), and the second wave of the SIMD fills
+// what is left (4 waves of 64x64, one per SIMD, read a quarter less from LDS but
+// took 13.28 us against 12.45 at 2048^3, 19.29 against 17.05 at 512x4096x4096, 30.6
+// against 26.8 at 1024x2048x7168).  A 4-deep LDS ring fed by buffer->LDS DMA keeps
+// three K steps (96 KiB per CU) in flight (a fifth stage measured slower).  The
+// 2048^3 GEMM (config 1) is 256 such tiles, one per CU, where the 256x256 kernel has
+// 64.
 #pragma once
 
 #include "gemm_fp8.hpp"
@@ -18,7 +22,7 @@
 namespace hkmoe {
 
 constexpr int kSmTile = 128;                         // output tile edge
-constexpr int kSmThreads = 256;                      // 4 waves
+constexpr int kSmThreads = 512;                      // 8 waves, two per SIMD
 constexpr int kSmStages = 4;                         // LDS ring depth (K steps)
 constexpr int kSmAhead = kSmStages - 1;              // K steps in flight beyond the current one
 constexpr int kSmOperandBytes = kSmTile * kBK;       // 16 KiB per operand per step
@@ -56,16 +60,16 @@ static_assert(kSmAhead <= 4, "small_wait_stage covers at most 3 newer stages");
 // order); a K step's words of the tile (64 per 64-row group of A and of B)
 // ride in the stage, one 4-byte-per-lane DMA per wave.
 template <bool F32OUT, bool M32, bool MX = false>
-__global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams p) {
+__global__ __launch_bounds__(kSmThreads, 2) void gemm_fp8_small(SmallGemmParams p) {
   static_assert(!(M32 && MX), "MX runs on the 16x16x128 MFMA");
   constexpr int kStg = sm_stage_bytes(MX);
-  constexpr int kLoads = MX ? 9 : 8;  // vector-memory instructions per wave and step
+  constexpr int kLoads = MX ? 5 : 4;  // vector-memory instructions per wave and step
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int l16 = lane & 15, lg = lane >> 4;
-  const int wm = wave >> 1, wn = wave & 1;  // the wave's 64x64 quarter
+  const int wm = wave >> 2, wn = wave & 3;  // the wave's 64 rows and 32 columns
   const int fx = swz(l16);
 
   // Tile of this workgroup.  Workgroups are dispatched round-robin over the 8
@@ -81,38 +85,40 @@ __global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams 
   const int m0 = mt * kSmTile, n0 = nt * kSmTile;
   const int k_steps = p.k / kBK;
 
-  // DMA: instruction i of wave w fills LDS rows 32i + 8w + lane/8 of an operand
+  // DMA: instruction i of wave w fills LDS rows 64i + 8w + lane/8 of an operand
   // tile; the lane fetches logical chunk (lane & 7) ^ swz(row), which lands
   // swizzled.  A rows past M repeat row M-1 (never stored).
   const int ld_row = 8 * wave + (lane >> 3);
   const int ld_chunk = (lane & 7) ^ swz(ld_row);
   const i32x4 a_srd = make_srd(p.a, p.a_bytes);
   const i32x4 b_srd = make_srd(p.b, p.b_bytes);
-  int a_voff[4], b_voff[4];
+  int a_voff[2], b_voff[2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int ra = min(m0 + 32 * i + ld_row, p.m - 1);
+  for (int i = 0; i < 2; ++i) {
+    const int ra = min(m0 + 64 * i + ld_row, p.m - 1);
     a_voff[i] = buf_off(ra, p.k, ld_chunk * 16);
-    b_voff[i] = buf_off(n0 + 32 * i + ld_row, p.k, ld_chunk * 16);
+    b_voff[i] = buf_off(n0 + 64 * i + ld_row, p.k, ld_chunk * 16);
   }
   // MX: waves 0, 1 fetch the words of A's two 64-row groups (a group past the
-  // padded rows repeats the last one: its rows are never stored), 2, 3 B's
-  const i32x4 w_srd = make_srd(wave < 2 ? p.a_scale : p.b_scale, 0xffffffffu);
-  const int w_voff = ((wave < 2 ? min(m0 + 64 * wave, p.m64 - 64) : n0 + 64 * (wave - 2)) + lane) * 4;
-  const int w_step = (wave < 2 ? p.m64 : p.n) * 4;
+  // padded rows repeats the last one: its rows are never stored), 2, 3 B's; 4-7
+  // repeat them, so that every wave has the same number of loads in flight
+  const int ww = wave & 3;
+  const i32x4 w_srd = make_srd(ww < 2 ? p.a_scale : p.b_scale, 0xffffffffu);
+  const int w_voff = ((ww < 2 ? min(m0 + 64 * ww, p.m64 - 64) : n0 + 64 * (ww - 2)) + lane) * 4;
+  const int w_step = (ww < 2 ? p.m64 : p.n) * 4;
   auto issue = [&](int kt) __attribute__((always_inline)) {
     uint8_t* st = smem + (kt % kSmStages) * kStg;
-    if constexpr (MX) load_lds_4B(w_srd, st + kSmStageBytes + wave * 256, w_voff, kt * w_step);
+    if constexpr (MX) load_lds_4B(w_srd, st + kSmStageBytes + ww * 256, w_voff, buf_off(kt, w_step, 0));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) load_lds_16B(a_srd, st + (32 * i + 8 * wave) * kBK, a_voff[i], kt * kBK);
+    for (int i = 0; i < 2; ++i) load_lds_16B(a_srd, st + (64 * i + 8 * wave) * kBK, a_voff[i], kt * kBK);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      load_lds_16B(b_srd, st + kSmOperandBytes + (32 * i + 8 * wave) * kBK, b_voff[i], kt * kBK);
+    for (int i = 0; i < 2; ++i)
+      load_lds_16B(b_srd, st + kSmOperandBytes + (64 * i + 8 * wave) * kBK, b_voff[i], kt * kBK);
   };
   // The wave's fragments of step kt.  16x16x128: A sub-tiles (rows 64wm + 16i
-  // + l16) and B fragments (columns 64wn + 16j + l16), K bytes 32lg .. +31.
-  // M32: fragment 2b + h is 32-row block b (rows 64wm + 32b + l32 of A, 64wn +
-  // 32b + l32 of B) and K half h: bytes 64h + 32g .. +31 (g = lane / 32), i.e.
+  // + l16) and B fragments (columns 32wn + 16j + l16), K bytes 32lg .. +31.
+  // M32: fragment 2b + h is 32-row block b (rows 64wm + 32b + l32 of A, 32wn +
+  // l32 of B) and K half h: bytes 64h + 32g .. +31 (g = lane / 32), i.e.
   // the 32-byte chunk pair 2h + g of the row; the rows of a block start at a
   // multiple of 32, so the swizzle of row l32 is the lane constant f32.
   const int l32 = lane & 31, g32 = lane >> 5;
@@ -120,63 +126,62 @@ __global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams 
   struct Words {
     int a, b;
   };
-  auto read = [&](int kt, i32x8 (&af)[4], i32x8 (&bf)[4], Words& w) __attribute__((always_inline)) {
+  auto read = [&](int kt, i32x8 (&af)[4], i32x8 (&bf)[2], Words& w) __attribute__((always_inline)) {
     const uint8_t* st = smem + (kt % kSmStages) * kStg;
     if constexpr (MX) {
       const int32_t* words = reinterpret_cast<const int32_t*>(st + kSmStageBytes);
       w.a = words[wm * 64 + lane];
-      w.b = words[kSmTile + wn * 64 + lane];
+      w.b = words[kSmTile + (wn >> 1) * 64 + lane] >> (16 * (wn & 1));
     }
     if constexpr (M32) {
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        af[f] = read_frag(st, 64 * wm + 32 * (f >> 1) + l32, 2 * (f & 1) + g32, f32);
-        bf[f] = read_frag(st + kSmOperandBytes, 64 * wn + 32 * (f >> 1) + l32, 2 * (f & 1) + g32, f32);
-      }
+      for (int f = 0; f < 4; ++f) af[f] = read_frag(st, 64 * wm + 32 * (f >> 1) + l32, 2 * (f & 1) + g32, f32);
+#pragma unroll
+      for (int f = 0; f < 2; ++f) bf[f] = read_frag(st + kSmOperandBytes, 32 * wn + l32, 2 * f + g32, f32);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) af[i] = read_operand<MX>(st, 64 * wm + 16 * i + l16, lg, fx);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) bf[j] = read_operand<MX>(st + kSmOperandBytes, 64 * wn + 16 * j + l16, lg, fx);
+      for (int j = 0; j < 2; ++j) bf[j] = read_operand<MX>(st + kSmOperandBytes, 32 * wn + 16 * j + l16, lg, fx);
     }
   };
 
-  // accumulators: 16x16x128: acc[i][j] (4 values); M32: acc32[bi][bj] (16 values)
-  f32x4 acc[4][4];
-  f32x16 acc32[2][2];
+  // accumulators: 16x16x128: acc[i][j] (4 values); M32: acc32[bi] (16 values)
+  f32x4 acc[4][2];
+  f32x16 acc32[2];
   if constexpr (M32) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc32[i][j][r] = 0.f;
+      for (int r = 0; r < 16; ++r) acc32[i][r] = 0.f;
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  auto mma = [&](const i32x8 (&af)[4], const i32x8 (&bf)[4], const Words& w) __attribute__((always_inline)) {
+  auto mma = [&](const i32x8 (&af)[4], const i32x8 (&bf)[2], const Words& w) __attribute__((always_inline)) {
     if constexpr (MX) {
-      mx_subtile<0>(acc[0], bf, af[0], w.b, w.a);
-      mx_subtile<1>(acc[1], bf, af[1], w.b, w.a);
-      mx_subtile<2>(acc[2], bf, af[2], w.b, w.a);
-      mx_subtile<3>(acc[3], bf, af[3], w.b, w.a);
+      auto sub = [&](auto u) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value;
+        acc[U][0] = mfma_mx<0, U>(bf[0], af[U], acc[U][0], w.b, w.a);
+        acc[U][1] = mfma_mx<1, U>(bf[1], af[U], acc[U][1], w.b, w.a);
+      };
+      sub(std::integral_constant<int, 0>{});
+      sub(std::integral_constant<int, 1>{});
+      sub(std::integral_constant<int, 2>{});
+      sub(std::integral_constant<int, 3>{});
     } else if constexpr (M32) {
-      // both K halves of the four blocks; a block's second MFMA is issued three
-      // MFMAs after its first
+      // both K halves of the two blocks
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc32[i][j] = mfma_e4m3_32x32x64(bf[2 * j + h], af[2 * i + h], acc32[i][j]);
+        for (int i = 0; i < 2; ++i) acc32[i] = mfma_e4m3_32x32x64(bf[h], af[2 * i + h], acc32[i]);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_e4m3_16x16x128(bf[j], af[i], acc[i][j]);
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma_e4m3_16x16x128(bf[j], af[i], acc[i][j]);
     }
   };
 
@@ -184,7 +189,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams 
   const int pre = min(kSmAhead, k_steps);
   for (int kt = 0; kt < pre; ++kt) issue(kt);
   small_wait_stage<kLoads>(pre - 1);
-  i32x8 af0[4], bf0[4], af1[4], bf1[4];
+  i32x8 af0[4], bf0[2], af1[4], bf1[2];
   Words w0{}, w1{};
   read(0, af0, bf0, w0);
 
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams 
   // iteration kt-2, complete at iteration kt-1's barrier); wait for step kt+1;
   // read its fragments into the other register set while the MFMAs of step kt
   // run.
-  auto step = [&](int kt, i32x8 (&ca)[4], i32x8 (&cb)[4], Words& cw, i32x8 (&na)[4], i32x8 (&nb)[4], Words& nw)
+  auto step = [&](int kt, i32x8 (&ca)[4], i32x8 (&cb)[2], Words& cw, i32x8 (&na)[4], i32x8 (&nb)[2], Words& nw)
       __attribute__((always_inline)) {
     if (kt + kSmAhead < k_steps) issue(kt + kSmAhead);
     if (kt + 1 < k_steps) {
@@ -209,7 +214,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams 
   // newer steps in flight.  (Written with the tail's conditions, the two
   // register sets got merged into one, which put each step's reads right
   // before its own MFMAs.)
-  auto step_full = [&](int kt, i32x8 (&ca)[4], i32x8 (&cb)[4], Words& cw, i32x8 (&na)[4], i32x8 (&nb)[4], Words& nw)
+  auto step_full = [&](int kt, i32x8 (&ca)[4], i32x8 (&cb)[2], Words& cw, i32x8 (&na)[4], i32x8 (&nb)[2], Words& nw)
       __attribute__((always_inline)) {
     issue(kt + kSmAhead);
     small_wait_stage<kLoads>(kSmAhead - 1);
@@ -229,62 +234,30 @@ __global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams 
   }
   if (kt < k_steps) step(kt, af0, bf0, w0, af1, bf1, w1);
 
-  // ---- epilogue: lane holds row 64wm + 16i + l16, columns 64wn + 16j + 4lg .. +3
-  // (M32: row 64wm + 32bi + l32, columns 64wn + 32bj + 8q + 4g32 .. +3 in
-  // registers 4q .. 4q+3 of acc32[bi][bj])
+  // ---- epilogue: lane holds row 64wm + 16i + l16, columns 32wn + 16j + 4lg .. +3
+  // (M32: row 64wm + 32bi + l32, columns 32wn + 8q + 4g32 .. +3 in registers
+  // 4q .. 4q+3 of acc32[bi])
   const float tens = MX ? 1.0f : (p.a_scale ? p.a_scale[0] : 1.0f) * (p.b_scale ? p.b_scale[0] : 1.0f);
-  if constexpr (M32 && F32OUT) {
+  constexpr int kRowSteps = M32 ? 2 : 4, kColSteps = M32 ? 4 : 2;
+  const int er = M32 ? l32 : l16;                     // row within a row step
+  auto value = [&](int i, int j) __attribute__((always_inline)) -> f32x4 {  // row step i, 4 columns j
+    if constexpr (M32)
+      return f32x4{acc32[i][4 * j], acc32[i][4 * j + 1], acc32[i][4 * j + 2], acc32[i][4 * j + 3]};
+    else
+      return acc[i][j];
+  };
+  if constexpr (F32OUT) {
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi) {
-      const int r = m0 + 64 * wm + 32 * bi + l32;
+    for (int i = 0; i < kRowSteps; ++i) {
+      const int r = m0 + 64 * wm + (64 / kRowSteps) * i + er;
       if (r < p.m) {
+        float* dst = static_cast<float*>(p.c) + static_cast<int64_t>(r) * p.n + n0 + 32 * wn + 4 * (M32 ? g32 : lg);
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj) {
-          float* dst = static_cast<float*>(p.c) + static_cast<int64_t>(r) * p.n + n0 + 64 * wn + 32 * bj + 4 * g32;
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<float4*>(dst + 8 * q) =
-                float4{acc32[bi][bj][4 * q] * tens, acc32[bi][bj][4 * q + 1] * tens,
-                       acc32[bi][bj][4 * q + 2] * tens, acc32[bi][bj][4 * q + 3] * tens};
+        for (int j = 0; j < kColSteps; ++j) {
+          const f32x4 v = value(i, j);
+          *reinterpret_cast<float4*>(dst + (32 / kColSteps) * j) =
+              float4{v.x * tens, v.y * tens, v.z * tens, v.w * tens};
         }
-      }
-    }
-  } else if constexpr (M32) {
-    // staged as below: row r, 16-byte chunk c = 8wn + 4bj + q, 8-byte half g32
-    __syncthreads();  // every wave is done with the ring
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi) {
-      const int r = 64 * wm + 32 * bi + l32;
-#pragma unroll
-      for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int c = 8 * wn + 4 * bj + q;
-          uint2 v;
-          v.x = pack_bf16x2(acc32[bi][bj][4 * q] * tens, acc32[bi][bj][4 * q + 1] * tens);
-          v.y = pack_bf16x2(acc32[bi][bj][4 * q + 2] * tens, acc32[bi][bj][4 * q + 3] * tens);
-          *reinterpret_cast<uint2*>(smem + r * 256 + ((c ^ (r & 15)) << 4) + g32 * 8) = v;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int idx = tid + kSmThreads * u, r = idx >> 4, c = idx & 15;
-      if (m0 + r < p.m) {
-        const uint4 v = *reinterpret_cast<const uint4*>(smem + r * 256 + ((c ^ (r & 15)) << 4));
-        *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.c) + static_cast<int64_t>(m0 + r) * p.n + n0 + c * 8) = v;
-      }
-    }
-  } else if constexpr (F32OUT) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = m0 + 64 * wm + 16 * i + l16;
-      if (r < p.m) {
-        float* dst = static_cast<float*>(p.c) + static_cast<int64_t>(r) * p.n + n0 + 64 * wn + 4 * lg;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          *reinterpret_cast<float4*>(dst + 16 * j) =
-              float4{acc[i][j][0] * tens, acc[i][j][1] * tens, acc[i][j][2] * tens, acc[i][j][3] * tens};
       }
     }
   } else {
@@ -292,20 +265,21 @@ __global__ __launch_bounds__(kSmThreads, 1) void gemm_fp8_small(SmallGemmParams 
     // c ^ (r & 15)) and stored as 16-byte chunks covering whole rows
     __syncthreads();  // every wave is done with the ring
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 64 * wm + 16 * i + l16;
+    for (int i = 0; i < kRowSteps; ++i) {
+      const int r = 64 * wm + (64 / kRowSteps) * i + er;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = 8 * wn + 2 * j + (lg >> 1);
+      for (int j = 0; j < kColSteps; ++j) {
+        const int c = 4 * wn + (M32 ? j : 2 * j + (lg >> 1)), half = M32 ? g32 : (lg & 1);
+        const f32x4 a = value(i, j);
         uint2 v;
-        v.x = pack_bf16x2(acc[i][j][0] * tens, acc[i][j][1] * tens);
-        v.y = pack_bf16x2(acc[i][j][2] * tens, acc[i][j][3] * tens);
-        *reinterpret_cast<uint2*>(smem + r * 256 + ((c ^ (r & 15)) << 4) + (lg & 1) * 8) = v;
+        v.x = pack_bf16x2(a.x * tens, a.y * tens);
+        v.y = pack_bf16x2(a.z * tens, a.w * tens);
+        *reinterpret_cast<uint2*>(smem + r * 256 + ((c ^ (r & 15)) << 4) + half * 8) = v;
       }
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < kSmTile * 16 / kSmThreads; ++u) {
       const int idx = tid + kSmThreads * u, r = idx >> 4, c = idx & 15;
       if (m0 + r < p.m) {
         const uint4 v = *reinterpret_cast<const uint4*>(smem + r * 256 + ((c ^ (r & 15)) << 4));
