@@ -597,8 +597,8 @@ def _kernel_label(name, dense=False):
         return "grouped_gemm1" if epi in "234" else "grouped_gemm2"
     if "gemm_fp8_narrow" in name:
         epi = name.split("Epi)")[1][0] if "Epi)" in name else "?"
-        return "narrow_gemm1" if epi == "3" else "narrow_gemm2"
-    if "gemm_fp8_small" in name:  # the dense GEMM's 128x128-tile kernel
+        return "narrow_gemm1" if epi in "234" else "narrow_gemm2"
+    if "gemm_fp8_small" in name or "gemm_fp8_skinny" in name:  # dense: 128x128 tiles, split-K strips
         return "gemm"
     n = name[len("void "):] if name.startswith("void ") else name  # template kernels
     if n.startswith("hkmoe::"):
@@ -649,16 +649,15 @@ def _write_timeline(f, path, n_calls):
         return
     with open(path) as tf:
         ks = sorted(csv.DictReader(tf), key=lambda r: int(r["Start_Timestamp"]))
-    starts = [i for i, r in enumerate(ks) if "route_topk" in r["Kernel_Name"]]
+    starts = [i for i, r in enumerate(ks) if "route_topk" in r["Kernel_Name"] or "route_small" in r["Kernel_Name"]]
     if len(starts) < n_calls:
         return
     i0 = starts[n_calls - 1]
     i1 = starts[n_calls] if len(starts) > n_calls else len(ks)
     t0 = int(ks[i0]["Start_Timestamp"])
-    f.write("\nTimeline of the last timed layer call (one `MoELayer` call: with block scales the narrow "
-            "kernels run on the library's auxiliary stream beside the 256x256 GEMMs, or, for decode-like "
-            "shapes with T*k <= E*64, on the same stream after each of them; per-tensor layers have no "
-            "narrow kernels):\n\n")
+    f.write("\nTimeline of the last timed layer call (one `MoELayer` call: narrow kernels, where the layer "
+            "has them, run on the library's auxiliary stream beside the 256x256 GEMMs, or, with few rows "
+            "per expert, on the same stream after each of them):\n\n")
     f.write("| kernel | start us | end us | duration us |\n|---|---|---|---|\n")
     for r in ks[i0:i1]:
         lab = _kernel_label(r["Kernel_Name"], False)
@@ -886,14 +885,14 @@ def summarize_counters(args):
 def layer_cus(cfg, device_cus=256, narrow_cus=64, max_rows=64):
     """CUs each kernel of a layer runs on, under the default narrow setting:
     with narrow experts (at most max_rows rows) beside larger ones and T*k >
-    2*E*max_rows (two-stream schedule) the first 256x256 GEMM keeps
-    device_cus - narrow_cus and the narrow GEMMs take narrow_cus; otherwise
-    (no narrow expert, the one-stream schedule, or the MX layer, which has no
-    narrow path) every kernel has every CU.  The routing is the benched one
+    2*E*max_rows (two-stream schedule; MX: T*k > 176*E, E >= 256 and at least
+    112 narrow experts) the first 256x256 GEMM keeps device_cus - narrow_cus and
+    the narrow GEMMs take narrow_cus; otherwise (no narrow expert, the one-stream
+    schedule) every kernel has every CU.  The routing is the benched one
     (host_draw), its top-k taken on the host (ties cannot occur on the drawn
     floats)."""
     import numpy as np
-    if cfg.get("mx") or not cfg["block"]:
+    if not (cfg.get("mx") or cfg["block"]):
         return {}
     _, logits = host_draw(cfg, 0)
     k, E = cfg["k"], cfg["E"]
@@ -901,6 +900,8 @@ def layer_cus(cfg, device_cus=256, narrow_cus=64, max_rows=64):
     counts = np.bincount(top.ravel(), minlength=E)
     narrow = int(((counts > 0) & (counts <= max_rows)).sum())
     if narrow == 0 or cfg["T"] * k <= 2 * E * max_rows:
+        return {}
+    if cfg.get("mx") and (E < 256 or narrow < 112 or cfg["T"] * k <= 176 * E):
         return {}
     return {"grouped_gemm1": device_cus - narrow_cus, "narrow_gemm1": narrow_cus, "narrow_gemm2": narrow_cus}
 

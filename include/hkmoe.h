@@ -291,11 +291,13 @@ size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t
  *     library-owned stream, beside the 256x256 kernels of the larger experts on the
  *     caller's stream, which waits for it before the combine.
  * Block-scaled layers with an even number of at most 64 128-wide K steps in both
- * GEMMs (H/128 and I/128) use it at every T; the others (per-tensor and MX scales,
- * other step counts) with at most max_rows tokens, where every expert is
- * narrow, or at least 256 experts.  Results are bit-identical with the narrow path
- * on or off.  cus == 0 turns it off; while 256x256 tiles exist the narrow kernels
- * take at most three quarters of the device's CUs, whatever cus asks for (the
+ * GEMMs (H/128 and I/128) use it at every T.  The others (per-tensor and MX scales,
+ * other step counts) use it with at most max_rows tokens, where every expert is
+ * narrow (row-major weights: up to 2.5 GB of them), and with packed weights of at
+ * least 256 experts, at least 112 of them narrow, on one stream up to T*top_k =
+ * 176*E (per-tensor: 256*E, and not above), then on the auxiliary one.  Results are
+ * bit-identical with the narrow path on or off.
+ * cus == 0 turns it off; while 256x256 tiles exist the narrow kernels take at most three quarters of the device's CUs, whatever cus asks for (the
  * first wide GEMM keeps the rest); wide_share 1 or 2 runs the first wide GEMM on
  * (CUs - cus) workgroups while narrow experts exist; with 2 the narrow path's CUs
  * also join that GEMM's remaining tiles once both narrow GEMMs are done (a second
@@ -365,10 +367,9 @@ int hkmoe_moe_forward(const void* x_q, const float* x_scale, const float* logits
  * I=2048, E=256, top-8, block scales), 856 for config-5 shapes (H=4096, I=1536,
  * E=128, top-8), 655 for config-2 shapes (H=4096, I=14336, E=8, top-2,
  * per-tensor scales).  Every kernel runs on `stream`: the narrow path's auxiliary
- * stream is not used, so block-scaled layers with T*k <= 2*E*max_rows (see
- * hkmoe_set_narrow; every layer of the three shapes above that fits the scratch)
- * take the one-stream narrow schedule, as hkmoe_moe_forward does, and larger
- * ones run the 256x256 kernels alone.  The first call on a device looks up that device's scratch
+ * stream is not used, so layers that hkmoe_moe_forward runs on one stream (see
+ * hkmoe_set_narrow; every layer of the first two shapes above that fits the scratch)
+ * take the same schedule here, and the rest run the 256x256 kernels alone.  The first call on a device looks up that device's scratch
  * address (hipGetSymbolAddress): make it outside graph capture.  All calls on
  * one device share its scratch and each call leaves its intermediates there:
  * calls that overlap in time on one device (other streams, other threads)
