@@ -477,30 +477,37 @@ int block_m_log2(int gemm) {
 
 // Per-device auxiliary stream (default priority, non-blocking) and fork/join
 // events of the one-call layer.  Created on the first call that is not being
-// captured into a graph; the mutex keeps fork/join sequences of concurrent
-// host threads from interleaving on the shared events.
+// captured into a graph.  g_aux_mu guards g_aux from that creation on and keeps
+// the fork/join sequences of concurrent host threads from interleaving on the shared
+// events: a call takes it before it looks at g_aux and holds it until it has
+// enqueued its join.
 struct AuxStreams {
   hipStream_t aux = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
-  bool ok = false;
 };
 std::mutex g_aux_mu;
 AuxStreams g_aux[kMaxDevices];
 
+// The current device's auxiliary stream (null: none); the caller holds g_aux_mu.
 int get_aux(hipStream_t main_stream, AuxStreams** out) {
   *out = nullptr;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return HKMOE_OK;
   AuxStreams& a = g_aux[dev];
-  if (!a.ok) {
+  if (a.aux == nullptr) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(main_stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
       return HKMOE_OK;  // no set-up under capture: this call runs without the narrow path
-    if (hipStreamCreateWithFlags(&a.aux, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&a.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&a.join, hipEventDisableTiming) != hipSuccess)
+    AuxStreams n;
+    if (hipStreamCreateWithFlags(&n.aux, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&n.fork, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&n.join, hipEventDisableTiming) != hipSuccess) {
+      if (n.fork) (void)hipEventDestroy(n.fork);
+      if (n.aux) (void)hipStreamDestroy(n.aux);
+      (void)hipGetLastError();  // reported here, not by a later launch
       return fail(HKMOE_ERR_HIP, "moe_forward: cannot create the auxiliary stream / events");
-    a.ok = true;
+    }
+    a = n;
   }
   *out = &a;
   return HKMOE_OK;
@@ -1081,7 +1088,7 @@ struct NarrowPlan {
   bool seq = false;
   int min_experts = 0;  // with fewer small experts the 256x256 kernels take them all
   AuxStreams* aux = nullptr;
-  std::unique_lock<std::mutex> lock;  // held while the fork / join is enqueued
+  std::unique_lock<std::mutex> lock;  // of g_aux_mu, held with aux until the join is enqueued
   bool on() const { return seq || aux != nullptr; }
 };
 
@@ -1129,9 +1136,10 @@ static int plan_narrow(const NarrowCall& c, hipStream_t s, NarrowPlan* plan) {
     plan->seq = c.rows <= c.experts * (c.tensor ? kMixedTensorRows : kMixedSeqRows);
   }
   if (plan->seq || !c.aux_ok) return HKMOE_OK;
-  HK_TRY(get_aux(s, &plan->aux));
-  if (plan->aux) plan->lock = std::unique_lock<std::mutex>(g_aux_mu);
-  return HKMOE_OK;
+  plan->lock = std::unique_lock<std::mutex>(g_aux_mu);
+  const int rc = get_aux(s, &plan->aux);
+  if (plan->aux == nullptr) plan->lock.unlock();
+  return rc;
 }
 
 // Routing, permutation, both grouped GEMMs and the combine, enqueued by `plan`.
