@@ -35,21 +35,24 @@ struct DType {
   bool operator!=(const char* o) const { return !(*this == o); }
 };
 
-// Tensor sizes: inline, since a call reads up to nine tensors.
+// Tensor sizes: inline, since a call reads up to nine tensors; more than
+// kInline of them all move to `rest`.
 struct Shape {
-  static constexpr size_t kMax = 16;
-  int64_t d[kMax];
+  static constexpr size_t kInline = 8;
+  int64_t d[kInline];
+  std::vector<int64_t> rest;
   size_t n = 0;
   size_t size() const { return n; }
-  int64_t operator[](size_t i) const { return d[i]; }
-  int64_t back() const { return d[n - 1]; }
-  const int64_t* begin() const { return d; }
-  const int64_t* end() const { return d + n; }
+  int64_t operator[](size_t i) const { return begin()[i]; }
+  int64_t back() const { return begin()[n - 1]; }
+  const int64_t* begin() const { return n <= kInline ? d : rest.data(); }
+  const int64_t* end() const { return begin() + n; }
   bool operator==(const Shape& o) const { return n == o.n && std::equal(begin(), end(), o.begin()); }
   bool operator!=(const Shape& o) const { return !(*this == o); }
   void push_back(int64_t v) {
-    if (n == kMax) throw std::runtime_error("tensor has too many dimensions");
-    d[n++] = v;
+    if (n == kInline) rest.assign(d, d + n);
+    if (n < kInline) d[n] = v; else rest.push_back(v);
+    ++n;
   }
 };
 

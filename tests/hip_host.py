@@ -60,3 +60,24 @@ def run(fake_dir, snippet, timeout=60):
                          env=env, timeout=timeout)
     assert res.returncode == 0, res.stdout[-3000:] + res.stderr[-3000:]
     return res.stdout.split("\n")[:-1]
+
+
+# tk_kernel over the stand-in runtime: torch is a stand-in too (the real one would
+# load its own HIP libraries), Tensor a class with the attributes the binding reads.
+BINDING = f"""
+import builtins, sys, time, types
+torch = types.ModuleType("torch")
+class Tensor:
+    def __init__(self, shape, dtype="torch.float32", device="cuda"):
+        self.shape, self.dtype, self.device = tuple(shape), dtype, types.SimpleNamespace(type=device)
+        self.is_cpu = device == "cpu"
+    def is_contiguous(self):
+        return True
+    def data_ptr(self):
+        return 1 << 20
+torch.Tensor, torch._C = Tensor, types.SimpleNamespace()
+torch.cuda = types.SimpleNamespace(current_stream=lambda: types.SimpleNamespace(cuda_stream=7))
+sys.modules["torch"] = torch
+sys.path.insert(0, {os.path.dirname(LIB)!r})
+import tk_kernel
+"""
