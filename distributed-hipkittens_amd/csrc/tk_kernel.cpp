@@ -18,6 +18,7 @@
 #include <cstdint>
 #include <cstring>
 #include <deque>
+#include <memory>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -90,6 +91,9 @@ py::object steal(PyObject* o) {
 }
 
 // Attribute names, torch.Tensor and the current-stream lookup, resolved once.
+// Not in a guarded static: the lookup runs Python code, which may hand the GIL to
+// a thread that then waits for the guard with the GIL held, for good.  Threads that
+// get here together each build their own and the first one to finish is kept.
 struct Names {
   PyObject *is_contiguous, *is_cpu, *data_ptr, *shape, *dtype;
   PyObject* tensor_type;
@@ -97,24 +101,24 @@ struct Names {
   py::object torch_cuda;
 };
 const Names& names() {
-  static const Names* n = [] {
-    auto* v = new Names();  // leaked, as above
-    v->is_contiguous = PyUnicode_InternFromString("is_contiguous");
-    v->is_cpu = PyUnicode_InternFromString("is_cpu");
-    v->data_ptr = PyUnicode_InternFromString("data_ptr");
-    v->shape = PyUnicode_InternFromString("shape");
-    v->dtype = PyUnicode_InternFromString("dtype");
-    py::module_ torch = py::module_::import("torch");
-    v->tensor_type = py::object(torch.attr("Tensor")).release().ptr();
-    v->torch_cuda = torch.attr("cuda");
-    py::object c = torch.attr("_C");
-    if (py::hasattr(c, "_cuda_getDevice") && py::hasattr(c, "_cuda_getCurrentRawStream")) {
-      v->get_device = py::object(c.attr("_cuda_getDevice")).release().ptr();
-      v->raw_stream = py::object(c.attr("_cuda_getCurrentRawStream")).release().ptr();
-    }
-    return v;
-  }();
-  return *n;
+  static const Names* kept = nullptr;  // read and written with the GIL held; leaked, as above
+  if (kept != nullptr) return *kept;
+  auto v = std::make_unique<Names>();
+  v->is_contiguous = PyUnicode_InternFromString("is_contiguous");
+  v->is_cpu = PyUnicode_InternFromString("is_cpu");
+  v->data_ptr = PyUnicode_InternFromString("data_ptr");
+  v->shape = PyUnicode_InternFromString("shape");
+  v->dtype = PyUnicode_InternFromString("dtype");
+  py::module_ torch = py::module_::import("torch");
+  v->tensor_type = py::object(torch.attr("Tensor")).release().ptr();
+  v->torch_cuda = torch.attr("cuda");
+  py::object c = torch.attr("_C");
+  if (py::hasattr(c, "_cuda_getDevice") && py::hasattr(c, "_cuda_getCurrentRawStream")) {
+    v->get_device = py::object(c.attr("_cuda_getDevice")).release().ptr();
+    v->raw_stream = py::object(c.attr("_cuda_getCurrentRawStream")).release().ptr();
+  }
+  if (kept == nullptr) kept = v.release();
+  return *kept;
 }
 
 // Plain torch.Tensor objects take the C API below (a tensor costs 0.3 us
