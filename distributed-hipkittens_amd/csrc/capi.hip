@@ -1149,7 +1149,7 @@ static int plan_narrow(const NarrowCall& c, hipStream_t s, NarrowPlan* plan) {
 extern "C++" {
 // route_topk, expert_offsets and scatter of at most kSmallTok tokens in one launch.
 static int launch_route_small(const float* logits, const MoeWorkspace& w, int64_t num_tokens, int32_t num_experts,
-                              int32_t top_k, int narrow_max, int32_t* narrow_info, hipStream_t s) {
+                              int32_t top_k, int narrow_max, int narrow_min, int32_t* narrow_info, hipStream_t s) {
   const int per_lane = (num_experts + 15) / 16;  // experts per lane of a token's 16-lane row
   auto kern = per_lane <= 1 ? route_small_kernel<1> : per_lane <= 2 ? route_small_kernel<2>
             : per_lane <= 4 ? route_small_kernel<4> : per_lane <= 8 ? route_small_kernel<8>
@@ -1157,7 +1157,7 @@ static int launch_route_small(const float* logits, const MoeWorkspace& w, int64_
                              : route_small_kernel<64>;
   hk_launch(kern, dim3(1), dim3(kScanThreads), 0, s, logits, static_cast<int>(num_tokens), num_experts, top_k,
             w.topk_idx, w.topk_w, w.counts, w.offsets, w.mtile_offsets, w.mtile_list, kBM, w.amax, w.tile_ctr,
-            narrow_max, narrow_info, w.perm, w.inv_perm);
+            narrow_max, narrow_min, narrow_info, w.perm, w.inv_perm);
   return check_launch("route_small_kernel");
 }
 
@@ -1171,7 +1171,7 @@ int moe_enqueue(const float* logits, const MoeWorkspace& w, int64_t num_tokens, 
   // (a timed call takes the three steps apart, so that each has a time of its own)
   if (num_tokens <= kSmallTok && !timed_call.on) {
     HK_TRY(launch_route_small(logits, w, num_tokens, num_experts, top_k, plan.on() ? nc.max_rows : 0,
-                              plan.on() ? w.narrow_info : nullptr, s));
+                              plan.min_experts, plan.on() ? w.narrow_info : nullptr, s));
   } else {
     HK_TRY(hkmoe_route_topk(logits, num_tokens, num_experts, top_k, w.topk_idx, w.topk_w, w.block_counts, s));
     t_role = HKMOE_TIMING_OFFSETS;

@@ -323,6 +323,12 @@ __device__ __forceinline__ int expert_offsets_tables(int e, int cnt, OffsetsLds&
   return off;
 }
 
+// Largest expert for the narrow kernel: narrow_max, or 0 (none) if fewer than
+// narrow_min experts are that small.  thread = expert; every thread calls it.
+__device__ __forceinline__ int narrow_limit(int cnt, int narrow_max, int narrow_min) {
+  return narrow_min > 0 && __syncthreads_count(cnt > 0 && cnt <= narrow_max) < narrow_min ? 0 : narrow_max;
+}
+
 __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
     int num_experts, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
     int32_t* __restrict__ mtile_offsets, int32_t* __restrict__ mtile_list, int tile_m,
@@ -349,8 +355,7 @@ __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
   } else if (e < num_experts) {
     cnt = counts[e];
   }
-  // fewer than narrow_min experts for the narrow kernel: none
-  if (narrow_min > 0 && __syncthreads_count(cnt > 0 && cnt <= narrow_max) < narrow_min) narrow_max = 0;
+  narrow_max = narrow_limit(cnt, narrow_max, narrow_min);
   expert_offsets_tables(e, cnt, lds, num_experts, offsets, mtile_offsets, mtile_list, tile_m, amax_reset,
                         tile_counters, narrow_max, narrow_info);
 }
@@ -368,7 +373,7 @@ __global__ __launch_bounds__(kScanThreads) void route_small_kernel(
     const float* __restrict__ logits, int num_tokens, int num_experts, int top_k, int32_t* __restrict__ topk_idx,
     float* __restrict__ topk_w, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
     int32_t* __restrict__ mtile_offsets, int32_t* __restrict__ mtile_list, int tile_m, float* amax_reset,
-    int32_t* tile_counters, int narrow_max, int32_t* narrow_info, int32_t* __restrict__ perm,
+    int32_t* tile_counters, int narrow_max, int narrow_min, int32_t* narrow_info, int32_t* __restrict__ perm,
     int32_t* __restrict__ inv_perm) {
   static_assert(kScanThreads == 16 * kSmallTok && kScanThreads >= kMaxExperts, "thread = token lane, then expert");
   __shared__ OffsetsLds lds;
@@ -386,6 +391,7 @@ __global__ __launch_bounds__(kScanThreads) void route_small_kernel(
   __syncthreads();
   const int cnt = tid < num_experts ? __popc(tokens[tid][0]) + __popc(tokens[tid][1]) : 0;
   if (tid < num_experts) counts[tid] = cnt;
+  narrow_max = narrow_limit(cnt, narrow_max, narrow_min);
   first[tid] = expert_offsets_tables(tid, cnt, lds, num_experts, offsets, mtile_offsets, mtile_list, tile_m, amax_reset,
                                      tile_counters, narrow_max, narrow_info);
   __syncthreads();

@@ -49,3 +49,35 @@ def test_topk_order_of_special_logits(hk, E, k):
     torch.cuda.synchronize()
     assert torch.equal(idx.cpu(), want)
     assert int(bc.sum()) == 40 * k
+
+
+@pytest.mark.parametrize("T", [24, 64, 65, 100])
+@pytest.mark.parametrize("hot", [True, False])
+def test_narrow_experts_of_few_tokens(hk, T, hot):
+    """MX layer of 256 experts with packed weights and the narrow limit at 16 rows.
+    A few small experts beside one that every token takes are not enough for the
+    narrow kernels, some 130 and more without a larger one are, whether routing is one
+    launch (T <= 64) or three."""
+    E, H, I, k = 256, 256, 128, 2 if hot else 8
+    gen = torch.Generator(device="cuda").manual_seed(T + k)
+    w13_q, w13_e = hk.quant_mx(torch.randn(E * 2 * I, H, device="cuda", generator=gen))
+    w2_q, w2_e = hk.quant_mx(torch.randn(E * H, I, device="cuda", generator=gen))
+    layer = hk.MoELayerMX(w13_q.view(E, 2 * I, H), w13_e.view(E, 2 * I, -1), w2_q.view(E, H, I), w2_e.view(E, H, -1), k)
+    x_q, x_e = hk.quant_mx(torch.randn(T, H, device="cuda", generator=gen))
+    logits = torch.randn(T, E, device="cuda", generator=gen)
+    logits[:, 7] += 30.0 if hot else 0.0
+    saved = hk.tk_kernel.get_narrow()
+    hk.tk_kernel.set_narrow(64, 16, 1)
+    try:
+        layer(x_q, x_e, logits)
+        torch.cuda.synchronize()
+    finally:
+        hk.tk_kernel.set_narrow(*saved)
+    counts = torch.bincount(torch.topk(logits, k, dim=1)[1].flatten(), minlength=E)
+    small = int(((counts > 0) & (counts <= 16)).sum())
+    assert bool((counts > 16).any()) == hot and (0 < small < 112) == hot
+    # the count of narrow experts, after the routing tables in the workspace
+    r, nblk = T * k, hk.tk_kernel.route_blocks(T)
+    sizes = [r, r, nblk * E, nblk * E, E, E + 1, E + 1, 2 * ((r + 255) // 256 + E), 1, 16]
+    at = sum((4 * n + 255) // 256 * 256 for n in sizes)
+    assert int(layer.workspace(T, "cuda")[at:at + 4].view(torch.int32)) == (0 if hot else small)
