@@ -886,7 +886,7 @@ def layer_cus(cfg, device_cus=256, narrow_cus=64, max_rows=64):
     """CUs each kernel of a layer runs on, under the default narrow setting:
     with narrow experts (at most max_rows rows) beside larger ones and T*k >
     2*E*max_rows (two-stream schedule; MX: T*k > 176*E, E >= 256 and at least
-    112 narrow experts) the first 256x256 GEMM keeps device_cus - narrow_cus and
+    100 narrow experts) the first 256x256 GEMM keeps device_cus - narrow_cus and
     the narrow GEMMs take narrow_cus; otherwise (no narrow expert, the one-stream
     schedule) every kernel has every CU.  The routing is the benched one
     (host_draw), its top-k taken on the host (ties cannot occur on the drawn
@@ -901,7 +901,7 @@ def layer_cus(cfg, device_cus=256, narrow_cus=64, max_rows=64):
     narrow = int(((counts > 0) & (counts <= max_rows)).sum())
     if narrow == 0 or cfg["T"] * k <= 2 * E * max_rows:
         return {}
-    if cfg.get("mx") and (E < 256 or narrow < 112 or cfg["T"] * k <= 176 * E):
+    if cfg.get("mx") and (E < 256 or narrow < 100 or cfg["T"] * k <= 176 * E):
         return {}
     return {"grouped_gemm1": device_cus - narrow_cus, "narrow_gemm1": narrow_cus, "narrow_gemm2": narrow_cus}
 

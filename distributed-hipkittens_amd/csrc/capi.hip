@@ -571,7 +571,7 @@ struct AuxJoin {
 int launch_expert_offsets(const int32_t* block_counts, int64_t num_tokens, int32_t num_experts,
                           int32_t* counts, int32_t* offsets, int32_t* block_base,
                           int32_t* mtile_offsets, int32_t* mtile_list, float* amax_reset,
-                          int32_t* tile_counters, int narrow_max, int narrow_min, int32_t* narrow_info,
+                          int32_t* tile_counters, int narrow_max, const NarrowRule& rule, int32_t* narrow_info,
                           hipStream_t stream) {
   const int nblk = route_blocks(num_tokens);
   // few routing blocks: expert_offsets_kernel also does the block scan (one
@@ -586,7 +586,7 @@ int launch_expert_offsets(const int32_t* block_counts, int64_t num_tokens, int32
     if (timed) t_role = HKMOE_TIMING_OFFSETS;
   }
   hk_launch(expert_offsets_kernel, dim3(1), dim3(kScanThreads), 0, stream, num_experts, counts, offsets,
-            mtile_offsets, mtile_list, kBM, amax_reset, tile_counters, narrow_max, narrow_min, narrow_info,
+            mtile_offsets, mtile_list, kBM, amax_reset, tile_counters, narrow_max, rule, narrow_info,
             block_counts, fuse ? nblk : -1, block_base);
   return check_launch("expert_offsets_kernel");
 }
@@ -676,7 +676,7 @@ int hkmoe_expert_offsets(const int32_t* block_counts, int64_t num_tokens, int32_
   HK_REQUIRE(num_tokens >= 0, "expert_offsets: bad T");
   HK_REQUIRE(num_tokens == 0 || block_counts, "expert_offsets: null block_counts");
   return launch_expert_offsets(block_counts, num_tokens, num_experts, counts, offsets, block_base,
-                               mtile_offsets, mtile_list, amax_reset, tile_counters, 0, 0, nullptr,
+                               mtile_offsets, mtile_list, amax_reset, tile_counters, 0, NarrowRule{}, nullptr,
                                static_cast<hipStream_t>(stream));
 }
 
@@ -694,7 +694,8 @@ int hkmoe_expert_offsets_narrow(const int32_t* block_counts, int64_t num_tokens,
   HK_REQUIRE(narrow_max >= 0 && narrow_max <= kNarrowRows, "expert_offsets_narrow: narrow_max=%d outside [0, %d]",
              narrow_max, kNarrowRows);
   return launch_expert_offsets(block_counts, num_tokens, num_experts, counts, offsets, block_base,
-                               mtile_offsets, mtile_list, amax_reset, tile_counters, narrow_max, 0, narrow_info,
+                               mtile_offsets, mtile_list, amax_reset, tile_counters, narrow_max, NarrowRule{},
+                               narrow_info,
                                static_cast<hipStream_t>(stream));
 }
 
@@ -1086,7 +1087,7 @@ size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t
 struct NarrowPlan {
   NarrowConfig cfg{};
   bool seq = false;
-  int min_experts = 0;  // with fewer small experts the 256x256 kernels take them all
+  NarrowRule rule;  // beside larger experts (narrow_limit); not met, the 256x256 kernels take all
   AuxStreams* aux = nullptr;
   std::unique_lock<std::mutex> lock;  // of g_aux_mu, held with aux until the join is enqueued
   bool on() const { return seq || aux != nullptr; }
@@ -1103,16 +1104,34 @@ struct NarrowPlan {
 //     Row-major weights, which the narrow kernel reads at 5.0-5.4 TB/s, only up to
 //     kRowMajorBytes of them (T=64 above: 498 -> 482 us; the 256x256 kernels reach
 //     5.9 on more: E=256 H=7168 I=2048 T=40 1376, narrow 1505 us);
-//   and packed ones from 256 experts on, where skewed routing leaves many small
-//     experts beside a few large: if at least kMixedExperts of them are small (the
-//     device decides; uniform T=2500, 15 small experts, lost 2%, skewed T=70, one
-//     expert above 64 rows beside 50, 5%).  H=7168 I=2048, skewed, per-tensor T=2000 /
-//     4000 / 8192 1484 / 2195 / 3488 -> 1435 / 2115 / 3404 us, uniform T=700 1959 ->
-//     1718.  MX on one stream up to kMixedSeqRows rows per expert (T=5000 2580 -> 2482
-//     us, on two 2654), on two above (T=6500 3175 -> 2786, on one 3034).  With fewer
-//     experts the two kernels one after the other lose what the smaller one gains: E=8
-//     per-tensor T=200 skewed 350 / 411 us, E=128 MX T=600 429 / 469 us.
-constexpr int kMixedExperts = 112;
+//   and with packed weights of at least 256 experts
+//     where no expert has more rows (the device decides): E=256 H=7168 I=2048
+//       per-tensor uniform T=700 1959 -> 1718 us, H=2048 I=768 MX T=400 320 -> 256,
+//       E=1024 H=1024 I=512 MX T=900 580 -> 383; 0.49 to 0.99 of the 256x256 kernels'
+//       time over 432 such batches;
+//     and beside larger experts, where the small ones pay (mixed_rule): on one stream
+//       if they save more than the second start and tail of each GEMM cost.  One saves
+//       0.25 us and 0.015 us per MB of its weights, less 0.002 us and 0.0004 us per MB
+//       for each row (per-tensor 0.36, 0.006, 0 and 0.0006): at 50-60 rows the narrow kernel
+//       gains little over a 256x256 tile.  MX T=4500: E=256 H=7168 I=2048 skewed, 118 small ones,
+//       2365 -> 2265 us; E=512 H=2048 I=512 uniform, 121 of 60 rows, would go 513 -> 553.
+//       On two streams at least 100 (108 to 147 gained 2-9%, whatever their size).
+//       Over 1224 batches (E = 256-1024, experts of 1.6-47 MB, T = 65-8192, uniform and
+//       skewed) those sent here took 1.02 of the 256x256 kernels' time at most; one
+//       number of small experts for all layers, 112, lost up to 9% on 87 of them.
+//       MX and block scales run on one stream up to kMixedSeqRows rows per expert (T=5000
+//       2580 -> 2482 us, on two 2654), on two above (T=6500 3175 -> 2786, on one 3034).
+//     Where neither holds, the empty narrow GEMMs take 4-6 us (on two streams 12).  Nothing
+//     is launched where not all experts can be small and more than half would have to pay.
+//   Fewer experts stay with the 256x256 kernels: uniform batches of E=128 and 192 would
+//     gain 10-15%, but small layers would pay those 4-6 us on every skewed one.
+static NarrowRule mixed_rule(int64_t expert_bytes, bool tensor, bool one_stream) {
+  if (!one_stream) return NarrowRule{100, 1, 0};
+  const double mb = 1e-6 * static_cast<double>(expert_bytes);
+  auto ns = [](double v) { return static_cast<int32_t>(v + 0.5); };
+  return tensor ? NarrowRule{40000, ns(360 + 6 * mb), ns(0.6 * mb)}
+                : NarrowRule{60000, ns(250 + 15 * mb), ns(2 + 0.4 * mb)};
+}
 constexpr int64_t kMixedSeqRows = 176, kMixedTensorRows = 256;
 constexpr int64_t kRowMajorBytes = 2500000000;
 struct NarrowCall {
@@ -1132,8 +1151,13 @@ static int plan_narrow(const NarrowCall& c, hipStream_t s, NarrowPlan* plan) {
     if (!plan->seq) return HKMOE_OK;
   } else {
     if (c.experts < 256 || !c.packed) return HKMOE_OK;
-    plan->min_experts = kMixedExperts;
     plan->seq = c.rows <= c.experts * (c.tensor ? kMixedTensorRows : kMixedSeqRows);
+    plan->rule = mixed_rule(c.expert_bytes, c.tensor, plan->seq);
+    if (plan->seq && c.rows > c.experts * max_rows &&
+        static_cast<int64_t>(c.experts) * plan->rule.per_expert < 2ll * plan->rule.need) {
+      plan->seq = false;
+      return HKMOE_OK;
+    }
   }
   if (plan->seq || !c.aux_ok) return HKMOE_OK;
   plan->lock = std::unique_lock<std::mutex>(g_aux_mu);
@@ -1149,7 +1173,8 @@ static int plan_narrow(const NarrowCall& c, hipStream_t s, NarrowPlan* plan) {
 extern "C++" {
 // route_topk, expert_offsets and scatter of at most kSmallTok tokens in one launch.
 static int launch_route_small(const float* logits, const MoeWorkspace& w, int64_t num_tokens, int32_t num_experts,
-                              int32_t top_k, int narrow_max, int narrow_min, int32_t* narrow_info, hipStream_t s) {
+                              int32_t top_k, int narrow_max, const NarrowRule& rule, int32_t* narrow_info,
+                              hipStream_t s) {
   const int per_lane = (num_experts + 15) / 16;  // experts per lane of a token's 16-lane row
   auto kern = per_lane <= 1 ? route_small_kernel<1> : per_lane <= 2 ? route_small_kernel<2>
             : per_lane <= 4 ? route_small_kernel<4> : per_lane <= 8 ? route_small_kernel<8>
@@ -1157,7 +1182,7 @@ static int launch_route_small(const float* logits, const MoeWorkspace& w, int64_
                              : route_small_kernel<64>;
   hk_launch(kern, dim3(1), dim3(kScanThreads), 0, s, logits, static_cast<int>(num_tokens), num_experts, top_k,
             w.topk_idx, w.topk_w, w.counts, w.offsets, w.mtile_offsets, w.mtile_list, kBM, w.amax, w.tile_ctr,
-            narrow_max, narrow_min, narrow_info, w.perm, w.inv_perm);
+            narrow_max, rule, narrow_info, w.perm, w.inv_perm);
   return check_launch("route_small_kernel");
 }
 
@@ -1171,13 +1196,13 @@ int moe_enqueue(const float* logits, const MoeWorkspace& w, int64_t num_tokens, 
   // (a timed call takes the three steps apart, so that each has a time of its own)
   if (num_tokens <= kSmallTok && !timed_call.on) {
     HK_TRY(launch_route_small(logits, w, num_tokens, num_experts, top_k, plan.on() ? nc.max_rows : 0,
-                              plan.min_experts, plan.on() ? w.narrow_info : nullptr, s));
+                              plan.rule, plan.on() ? w.narrow_info : nullptr, s));
   } else {
     HK_TRY(hkmoe_route_topk(logits, num_tokens, num_experts, top_k, w.topk_idx, w.topk_w, w.block_counts, s));
     t_role = HKMOE_TIMING_OFFSETS;
     HK_TRY(launch_expert_offsets(w.block_counts, num_tokens, num_experts, w.counts, w.offsets, w.block_base,
                                  w.mtile_offsets, w.mtile_list, w.amax, w.tile_ctr, plan.on() ? nc.max_rows : 0,
-                                 plan.min_experts, plan.on() ? w.narrow_info : nullptr, s));
+                                 plan.rule, plan.on() ? w.narrow_info : nullptr, s));
     t_role = HKMOE_TIMING_SCATTER;
     HK_TRY(hkmoe_scatter(w.topk_idx, num_tokens, num_experts, top_k, w.offsets, w.block_base, w.perm, w.inv_perm,
                          nullptr, nullptr, hidden, HKMOE_SCALE_TENSOR, nullptr, nullptr, s));

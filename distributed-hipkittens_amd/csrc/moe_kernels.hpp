@@ -323,16 +323,30 @@ __device__ __forceinline__ int expert_offsets_tables(int e, int cnt, OffsetsLds&
   return off;
 }
 
-// Largest expert for the narrow kernel: narrow_max, or 0 (none) if fewer than
-// narrow_min experts are that small.  thread = expert; every thread calls it.
-__device__ __forceinline__ int narrow_limit(int cnt, int narrow_max, int narrow_min) {
-  return narrow_min > 0 && __syncthreads_count(cnt > 0 && cnt <= narrow_max) < narrow_min ? 0 : narrow_max;
+// What small experts must save for the narrow kernels to take them beside larger
+// ones: per_expert less per_row per row each, need in all (ns).  need 0: no condition.
+struct NarrowRule {
+  int32_t need = 0, per_expert = 0, per_row = 0;
+};
+
+// Largest expert for the narrow kernel: narrow_max, or 0 (none) where an expert is
+// larger and the small ones do not save enough.  thread = expert; every thread calls it.
+__device__ __forceinline__ int narrow_limit(int cnt, int narrow_max, const NarrowRule& rule) {
+  __shared__ int saved;
+  if (threadIdx.x == 0) saved = 0;
+  if (rule.need <= 0 || !__syncthreads_or(cnt > narrow_max)) return narrow_max;
+  int v = cnt > 0 && cnt <= narrow_max ? rule.per_expert - rule.per_row * cnt : 0;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, kWave);
+  if ((threadIdx.x & 63) == 0) atomicAdd(&saved, v);
+  __syncthreads();
+  return saved >= rule.need ? narrow_max : 0;
 }
 
 __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
     int num_experts, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
     int32_t* __restrict__ mtile_offsets, int32_t* __restrict__ mtile_list, int tile_m,
-    float* amax_reset, int32_t* tile_counters, int narrow_max, int narrow_min, int32_t* narrow_info,
+    float* amax_reset, int32_t* tile_counters, int narrow_max, NarrowRule rule, int32_t* narrow_info,
     const int32_t* __restrict__ block_counts, int fused_nblk, int32_t* __restrict__ block_base) {
   __shared__ OffsetsLds lds;
   const int e = threadIdx.x;  // E <= kScanThreads
@@ -355,7 +369,7 @@ __global__ __launch_bounds__(kScanThreads) void expert_offsets_kernel(
   } else if (e < num_experts) {
     cnt = counts[e];
   }
-  narrow_max = narrow_limit(cnt, narrow_max, narrow_min);
+  narrow_max = narrow_limit(cnt, narrow_max, rule);
   expert_offsets_tables(e, cnt, lds, num_experts, offsets, mtile_offsets, mtile_list, tile_m, amax_reset,
                         tile_counters, narrow_max, narrow_info);
 }
@@ -373,7 +387,7 @@ __global__ __launch_bounds__(kScanThreads) void route_small_kernel(
     const float* __restrict__ logits, int num_tokens, int num_experts, int top_k, int32_t* __restrict__ topk_idx,
     float* __restrict__ topk_w, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
     int32_t* __restrict__ mtile_offsets, int32_t* __restrict__ mtile_list, int tile_m, float* amax_reset,
-    int32_t* tile_counters, int narrow_max, int narrow_min, int32_t* narrow_info, int32_t* __restrict__ perm,
+    int32_t* tile_counters, int narrow_max, NarrowRule rule, int32_t* narrow_info, int32_t* __restrict__ perm,
     int32_t* __restrict__ inv_perm) {
   static_assert(kScanThreads == 16 * kSmallTok && kScanThreads >= kMaxExperts, "thread = token lane, then expert");
   __shared__ OffsetsLds lds;
@@ -391,7 +405,7 @@ __global__ __launch_bounds__(kScanThreads) void route_small_kernel(
   __syncthreads();
   const int cnt = tid < num_experts ? __popc(tokens[tid][0]) + __popc(tokens[tid][1]) : 0;
   if (tid < num_experts) counts[tid] = cnt;
-  narrow_max = narrow_limit(cnt, narrow_max, narrow_min);
+  narrow_max = narrow_limit(cnt, narrow_max, rule);
   first[tid] = expert_offsets_tables(tid, cnt, lds, num_experts, offsets, mtile_offsets, mtile_list, tile_m, amax_reset,
                                      tile_counters, narrow_max, narrow_info);
   __syncthreads();

@@ -294,9 +294,11 @@ size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t
  * GEMMs (H/128 and I/128) use it at every T.  The others (per-tensor and MX scales,
  * other step counts) use it with at most max_rows tokens, where every expert is
  * narrow (row-major weights: up to 2.5 GB of them), and with packed weights of at
- * least 256 experts, at least 112 of them narrow, on one stream up to T*top_k =
- * 176*E (per-tensor: 256*E, and not above), then on the auxiliary one.  Results are
- * bit-identical with the narrow path on or off.
+ * least 256 experts where the routing leaves no expert above max_rows rows, or enough
+ * narrow ones beside the larger: on one stream, up to T*top_k = 176*E (per-tensor:
+ * 256*E, and not above), by an estimate of what they save (70 of 44 MB and 10 rows each
+ * are enough), then on the auxiliary one at least 100.  Results are bit-identical
+ * with the narrow path on or off.
  * cus == 0 turns it off; while 256x256 tiles exist the narrow kernels take at most three quarters of the device's CUs, whatever cus asks for (the
  * first wide GEMM keeps the rest); wide_share 1 or 2 runs the first wide GEMM on
  * (CUs - cus) workgroups while narrow experts exist; with 2 the narrow path's CUs

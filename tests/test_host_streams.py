@@ -14,7 +14,7 @@ def fake(tmp_path_factory):
     return hip_host.build_fake(str(tmp_path_factory.mktemp("fake_hip")))
 
 
-CALL = {"block": "moe(8192, 64, 4, 512, 256, BLOCK, 1, s)", "mx": "moe_mx(16384, 256, 4, 512, 256, 1, s)"}
+CALL = {"block": "moe(8192, 64, 4, 512, 256, BLOCK, 1, s)", "mx": "moe_mx(16384, 256, 4, 4096, 1536, 1, s)"}
 
 
 @pytest.mark.parametrize("call", list(CALL.values()), ids=list(CALL))
