@@ -226,10 +226,10 @@ int launch_gemm_skinny(SkinnyParams p, bool f32out, hipStream_t stream) {
 // Estimated times (us) of the dense kernels, from which the dense GEMM picks one:
 // rounds of workgroups over the CUs x (ramp + K steps x time per step), or B's
 // stream from HBM where that is longer (a tenth of the compute term breaks ties
-// there).  The constants are fits to graph-replayed launches with three operand
-// copies; on 90 other shapes (M = 24 .. 3333, N = 1024 .. 7168, K = 1536 .. 14336,
-// both outputs and modes) the pick costs 1.6% over the best kernel on average,
-// 11% at worst.
+// there).  The constants are fits to graph-replayed launches over rotating operand
+// copies: on 1040 shapes (M = 1 .. 12000, N = 256 .. 16384, K = 128 .. 14336, both outputs
+// and modes) the pick costs 0.8% over the best kernel on average; with one K step up to
+// 30% (1 us), else 17%.
 //   split-K strips against 128x128 tiles: 128x2048x8192 9.3 / 29.5 us, 128x8192x1024
 //     6.4 / 7.0, 512x2048x2048 8.2 / 10.4 (and losing: 512x4096x4096 20.8 / 17.3)
 //   128x128 against 256x256 tiles: 2048^3 13.9 / 25.6 us, 2048x4096x4096 40.8 / 48.1
@@ -265,18 +265,26 @@ DenseKernel pick_dense(int64_t m, int64_t n, int64_t k, bool f32out, bool mx) {
   };
   {
     const double tiles = static_cast<double>((m + kBM - 1) / kBM) * (n / kBN);
-    const double step = tiles <= cus / 4 ? (mx ? 1.12 : 0.95) : tiles <= cus / 2 ? (mx ? 1.27 : 1.13) : (mx ? 1.45 : 1.3);
+    auto step = [&](double t) {  // per step, t tiles in the round
+      return t <= cus / 4 ? (mx ? 1.12 : 0.95) : t <= cus / 2 ? (mx ? 1.27 : 1.13) : (mx ? 1.45 : 1.3);
+    };
     int64_t rounds;
     (void)dense_block_log2(m, n, &rounds);
-    offer(DenseKernel::kTile256, 5.4 + static_cast<double>(rounds) * ((f32out ? 11 : 5) + ks * step), 0);
+    const double full = static_cast<double>(rounds - 1), ramp = f32out ? 10 : 4.5;
+    const double last = rounds == 1 ? tiles : std::max(1.0, std::min(cus, tiles - full * cus));
+    offer(DenseKernel::kTile256, 5.4 + full * (ramp + ks * step(cus)) + ramp + ks * step(last), 0);
   }
   {
-    const uint64_t tiles = ((um + kSmTile - 1) / kSmTile) * (un / kSmTile);
+    // M tiles in fours: the workgroups that a 4x8 block has past M exit at once, but they
+    // take their turns in the dispatch, and the live ones share a part of the CUs
+    // (65x11264x2048, 88 live ones: 24 us, as two rounds would)
+    const uint64_t mt = (um + kSmTile - 1) / kSmTile, nt = un / kSmTile, tiles = (mt + 3) / 4 * 4 * nt;
     const double full = static_cast<double>(tiles / ncu), part = static_cast<double>(tiles % ncu);
+    const double live = std::min(part, static_cast<double>(mt * nt));  // of the last round
     const double busy = mx ? 0.58 : 0.52, idle = mx ? 0.51 : 0.40;  // per step, chip full / half full
-    const double ramp = f32out ? 4.8 : 2.3;
+    const double ramp = f32out ? 4.0 : 2.6;
     offer(DenseKernel::kTile128,
-          2 + full * (ramp + ks * busy) + (part > 0 ? ramp + ks * (part <= cus / 2 ? idle : busy) : 0), 3 + nk / 2.0e6);
+          1.75 + full * (ramp + ks * busy) + (part > 0 ? ramp + ks * (live <= cus / 2 ? idle : busy) : 0), 3 + nk / 2.0e6);
   }
   const struct {
     DenseKernel kern;
