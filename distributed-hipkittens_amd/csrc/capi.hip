@@ -1431,10 +1431,12 @@ int hkmoe_quant_mx(const float* x, int64_t rows, int64_t cols, void* q, void* s,
              (long long)cols);
   const int64_t blocks = rows * (cols / 32);
   if (blocks == 0) return HKMOE_OK;
-  const int64_t grid = (blocks * 8 + kMxQuads - 1) / kMxQuads;
+  const bool small = blocks * 32 <= kMxSmall;
+  const int64_t per = small ? 512 : 1024, grid = (blocks * 8 + per - 1) / per;  // quads per workgroup
   HK_REQUIRE(grid < (1ll << 31), "quant_mx: too large");
-  hipLaunchKernelGGL(quant_mx_kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), x, blocks, static_cast<uint8_t*>(q), static_cast<uint8_t*>(s));
+  hipLaunchKernelGGL((small ? quant_mx_kernel<2, false> : quant_mx_kernel<4, true>), dim3(static_cast<unsigned>(grid)),
+                     dim3(256), 0, static_cast<hipStream_t>(stream), x, blocks, static_cast<uint8_t*>(q),
+                     static_cast<uint8_t*>(s));
   return check_launch("quant_mx_kernel");
 }
 

@@ -888,22 +888,28 @@ __global__ __launch_bounds__(1024) void quant_tensor_small_kernel(const float* _
 // -- and q = e4m3(x * 2^(127 - s)), an exact power-of-two scaling followed by
 // one RNE conversion (|x * 2^(127-s)| < 2, so the saturating clamp never acts).
 // Reference behaviour: 4_wave.cu:296-321, 368-373.
-// Each workgroup owns 1024 quads; a thread's four loads are in flight together.
-constexpr int kMxQuads = 1024;
+// Each workgroup owns 256 U quads; a thread's U loads are in flight together.  Up to
+// kMxSmall values two loads, kept in the caches: fewer per thread spread a small
+// tensor over more CUs (64x4096 1.9 us, four loads 2.2), and x was written just
+// before it is quantised (1024x7168 with six inputs in turn 7.0 us, non-temporal
+// 7.9).  Above, four non-temporal ones (4096x7168 in turn 23.7 us, else 26.9).
+constexpr int64_t kMxSmall = 1 << 23;
+template <int U, bool NT>
 __global__ __launch_bounds__(256) void quant_mx_kernel(const float* __restrict__ x, int64_t blocks,
                                                        uint8_t* __restrict__ q, uint8_t* __restrict__ s) {
   const int64_t quads = blocks * 8;
   // quad i = lane i % 8 of block i / 8; the 8 lanes of a block sit in one DPP
   // row (i % 8 == threadIdx.x % 8) and are in or out of range together
-  const int64_t i0 = blockIdx.x * static_cast<int64_t>(kMxQuads) + threadIdx.x;
-  f32x4 v[4];
+  const int64_t i0 = blockIdx.x * static_cast<int64_t>(256 * U) + threadIdx.x;
+  f32x4 v[U];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
+    const f32x4_u* src = reinterpret_cast<const f32x4_u*>(x) + i0 + 256 * u;
     v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (i0 + 256 * u < quads) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(x) + i0 + 256 * u);
+    if (i0 + 256 * u < quads) v[u] = NT ? __builtin_nontemporal_load(src) : *src;
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int64_t i = i0 + 256 * u;
     float m = max_abs4(v[u]);
     m = fmaxf(m, __shfl_xor(m, 1, kWave));

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from helpers import f8_np
-from oracle import spec
+from oracle import mx, spec
 
 pytestmark = pytest.mark.gpu
 
@@ -100,3 +100,22 @@ def test_quantiser_non_finite(tk, what, shape):
         assert got[7] & 0x7F == 0x7F
         q_ref[7] = got[7]
         np.testing.assert_array_equal(got, q_ref)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (63, 32), (64, 32), (65, 32), (127, 160), (2048, 4096), (2049, 4096)])
+def test_quant_mx_edges(tk, rows, cols, off):
+    """MX: partial workgroups and both sides of the two kernels' line (2^23 values)."""
+    x = _data((rows, cols), seed=rows + off)
+    q_ref, s_ref = mx.quant_mx(x)
+    # what lies around the outputs must stay untouched
+    q_buf = torch.full((rows * cols + off + 64,), 0x55, dtype=torch.uint8, device="cuda")
+    s_buf = torch.full((rows * cols // 32 + 64,), 0x55, dtype=torch.uint8, device="cuda")
+    q = q_buf[off:off + rows * cols].view(torch.float8_e4m3fn).view(rows, cols)
+    s = s_buf[:rows * cols // 32].view(rows, cols // 32)
+    tk.dispatch_quant_mx(_at(x, off, torch.float32), q, s)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(f8_np(q), q_ref)
+    np.testing.assert_array_equal(s.cpu().numpy(), s_ref)
+    assert bool((q_buf[:off] == 0x55).all()) and bool((q_buf[off + rows * cols:] == 0x55).all())
+    assert bool((s_buf[rows * cols // 32:] == 0x55).all())
