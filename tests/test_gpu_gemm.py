@@ -31,7 +31,13 @@ def dense_mfma(hk, request):
     hk.tk_kernel.set_dense_mfma(saved)
 
 
-# all four shapes have fewer 256x256 tiles than two per CU: the 128x128 kernel
+# shapes of the 128x128 kernel (test_host_dense.py checks that they are): partial row
+# tiles, fewer K steps than its ring has stages, odd and even step counts, whole blocks
+SMALL_KERNEL = [(2048, 2048, 2048), (777, 2048, 640), (2001, 2048, 384), (1000, 4096, 256), (300, 16384, 128),
+                (257, 4096, 4096), (1100, 2304, 896)]
+
+
+# and, beside one of those, shapes that run in split-K strips, where the setting changes nothing
 @pytest.mark.parametrize("dense_mfma", [16, 32], indirect=True)
 @pytest.mark.parametrize("m,n,k", [(256, 256, 128), (512, 512, 1024), (2048, 2048, 2048), (77, 256, 384)])
 def test_pm1_known_answer_fp32(hk, dense_mfma, m, n, k):
@@ -48,10 +54,12 @@ def test_pm1_known_answer_fp32(hk, dense_mfma, m, n, k):
 
 
 @pytest.mark.parametrize("dense_mfma", [32], indirect=True)
-@pytest.mark.parametrize("m,n,k", [(1, 256, 128), (300, 768, 640), (2048, 2048, 2048)])
+@pytest.mark.parametrize("m,n,k", [(1, 256, 128), (300, 768, 640), (2048, 2048, 2048), (777, 2048, 640),
+                                   (1100, 2304, 896)])
 def test_gemm_mfma32_bf16(hk, dense_mfma, m, n, k):
     """The 32x32x64 kernel with scales and bf16 output against the oracle, and
-    against the 16x16x128 kernel's bf16 output (same fp32 sums up to order)."""
+    against the 16x16x128 kernel's bf16 output (same fp32 sums up to order).  The
+    first two shapes run in split-K strips with either setting."""
     d = synth.make_dense(m, n, k, seed=m + 1)
     ref = spec.gemm_fp8(d["a_q"], d["b_q"], d["sa"], d["sb"], out="f32")
     args = (to_f8(d["a_q"]), to_f8(d["b_q"]), to_f32([d["sa"]]), to_f32([d["sb"]]))
@@ -61,6 +69,22 @@ def test_gemm_mfma32_bf16(hk, dense_mfma, m, n, k):
     torch.cuda.synchronize()
     assert rel_err(bf16_np(c32), ref) <= TOL
     assert rel_err(bf16_np(c32), bf16_np(c16)) <= 8e-3
+
+
+@pytest.mark.parametrize("dense_mfma", [16, 32], indirect=True)
+@pytest.mark.parametrize("m,n,k", SMALL_KERNEL)
+def test_small_kernel_both_mfma_shapes(hk, dense_mfma, m, n, k):
+    """The 128x128 kernel with either MFMA shape: +-1 operands and scales of product
+    2, so every value is an exact integer; both outputs, and the row past the last."""
+    rng = np.random.default_rng(m + n + k)
+    a, b = to_f8(_pm1(rng, (m, k))), to_f8(_pm1(rng, (n, k)))
+    ref = 2.0 * (a.double() @ b.double().T)
+    for dtype in (torch.float32, torch.bfloat16):
+        buf = torch.full((m + 1, n), 7.0, dtype=dtype, device="cuda")
+        hk.tk_kernel.dispatch_gemm_fp8(a, b, buf[:m], to_f32([4.0]), to_f32([0.5]))
+        torch.cuda.synchronize()
+        assert torch.equal(buf[:m], ref.to(torch.float32).to(dtype))
+        assert bool((buf[m] == 7.0).all())
 
 
 def test_dispatch_micro_4d_views(hk):

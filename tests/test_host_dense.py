@@ -6,6 +6,8 @@ import re
 import pytest
 
 import hip_host
+import test_gpu_dense_shapes
+import test_gpu_gemm
 
 
 @pytest.fixture(scope="module")
@@ -13,19 +15,25 @@ def fake(tmp_path_factory):
     return hip_host.build_fake(str(tmp_path_factory.mktemp("fake_hip")))
 
 
-def kernels(fake, calls, mfma=32):
-    """The kernel of each (m, n, k, f32, mx): "strip <MF, NF, NW>", "128" or "256"."""
+def launches(fake, calls, mfma):
+    """The launch line of each (m, n, k, f32, mx)."""
     out = hip_host.run(fake, f"""
     assert lib.hkmoe_set_dense_mfma({mfma}) == 0
     for c in {calls!r}:
         assert dense(*c) == 0, lib.hkmoe_last_error()
     print(json.dumps(log()))
     """)
+    lines = json.loads(out[-1])
+    assert len(lines) == len(calls)
+    return lines
+
+
+def kernels(fake, calls, mfma=32):
+    """The kernel of each call: "strip MFxNF" (16 MF rows, 16 NF columns), "128" or "256"."""
     names = []
-    for line in json.loads(out[-1]):
+    for line in launches(fake, calls, mfma):
         m = re.match(r"launch hkmoe::gemm_fp8_(skinny<(\d), *_?(\d), *_?(\d)|small|persistent)", line)
         names.append(f"strip {m.group(2)}x{m.group(3)}" if m.group(2) else {"small": "128", "persistent": "256"}[m.group(1)])
-    assert len(names) == len(calls)
     return names
 
 
@@ -43,3 +51,31 @@ PICKS = [((2048, 2048, 2048, 0, 0), "128"), ((8192, 8192, 2048, 0, 0), "256"), (
 
 def test_picks(fake):
     assert kernels(fake, [c for c, _ in PICKS]) == [k for _, k in PICKS]
+
+
+def test_gpu_shapes_reach_every_kernel(fake):
+    """Every form of every dense kernel has a shape in the GPU test, and the 256x256
+    kernel each of its tile blocks (2^b M tiles x 2^(5-b) N tiles)."""
+    want = {"strip 1x1", "strip 2x1", "strip 1x2", "strip 2x2", "strip 2x4", "strip 4x4", "128", "256"}
+    for mx in (0, 1):
+        for f32 in (0, 1):
+            got = kernels(fake, [(m, n, k, f32, mx) for m, n, k in test_gpu_dense_shapes.SHAPES])
+            assert set(got) == want, (mx, f32, want - set(got))
+            blocks = set()
+            for (m, n, _), kern in zip(test_gpu_dense_shapes.SHAPES, got):
+                mt, nt = -(-m // 256), n // 256
+                rounds = lambda b: -(-(-(-mt // 2 ** b) * -(-nt // 2 ** (5 - b))) // 8)
+                if kern == "256":
+                    blocks.add(min((2, 3, 1, 4, 5, 0), key=rounds))
+            assert blocks >= {0, 2, 3, 4, 5} | ({1} if f32 == 0 else set()), blocks
+
+
+def test_mfma_shapes_of_the_128_kernel(fake):
+    """The GPU test's shapes of the 128x128 kernel run on it, on the MFMA asked for
+    (template arguments: fp32 output, 32x32x64, MX)."""
+    for mfma in (16, 32):
+        for f32 in (0, 1):
+            calls = [(m, n, k, f32, 0) for m, n, k in test_gpu_gemm.SMALL_KERNEL]
+            form = f"gemm_fp8_small<{'true' if f32 else 'false'},_{'true' if mfma == 32 else 'false'},_false>"
+            for c, line in zip(calls, launches(fake, calls, mfma)):
+                assert form in line, (c, line)
