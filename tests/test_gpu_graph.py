@@ -11,14 +11,17 @@ input set is replayed twice; between replays the test runs other eager work
 (copies, and an eager call of the same layer object, on the same workspace, on
 other inputs) and synchronises, and that eager result is checked as well.
 
-The narrow path (block scales, even H/128 and I/128) forks to the library's
-auxiliary stream and joins back through events; under capture the auxiliary
+The narrow path forks to the library's auxiliary stream and joins back through
+events (block scales with even H/128 and I/128; MX and other block-scaled layers
+with many experts, test_moe_layer_mx_two_streams); under capture the auxiliary
 stream joins the graph the same way, with the late join (wide_share 2) and
 without it (1).  Where T*k <= 2*E*max_rows it stays on the caller's stream,
 which the capture takes as it is.
 """
 import pytest
 import torch
+
+import test_gpu_narrow_modes
 
 pytestmark = pytest.mark.gpu
 
@@ -140,3 +143,29 @@ def test_moe_layer_graph_replay_narrow(hk, share, max_rows):
         _replay_and_check(layer, sets)
     finally:
         hk.tk_kernel.set_narrow(*saved)
+
+
+def test_moe_layer_mx_two_streams(hk):
+    """MX layer whose narrow kernels run on the auxiliary stream (6500 tokens, 256
+    experts of both kinds), captured: the fork and the join are in the graph.  And
+    timed (hkmoe_kernel_timing): the same bits, the narrow GEMMs beside the 256x256
+    GEMM 1 and joined before the combine."""
+    tk = hk.tk_kernel
+    layer = test_gpu_narrow_modes._large_layer(hk, "mx")
+    sets = [test_gpu_narrow_modes._large_inputs(hk, layer, "mx", 6500, seed) for seed in (1, 2)]
+    _replay_and_check(layer, sets)
+    want = layer(*sets[0]).clone()
+    tk.kernel_timing(1)
+    try:
+        out = layer(*sets[0])
+        torch.cuda.synchronize()
+        timeline = tk.kernel_timing_read(0)
+    finally:
+        tk.kernel_timing(0)
+    assert _same(out, want)
+    got = {tk.TIMING_ROLES[i]: v for i, v in enumerate(timeline) if v[0] >= 0}
+    print(f"MX two streams, timeline (ms): {got}", flush=True)
+    assert got["narrow_gemm1"][0] < got["grouped_gemm1"][1]
+    assert got["narrow_gemm1"][1] <= got["narrow_gemm2"][0] + 1e-3
+    assert got["narrow_gemm2"][1] <= got["combine"][0] + 1e-3
+    assert got["grouped_gemm2"][1] <= got["combine"][0] + 1e-3
