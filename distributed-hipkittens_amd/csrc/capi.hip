@@ -54,7 +54,8 @@ int check_launch(const char* what) {
 // on, each kernel a layer call enqueues is launched by hipExtLaunchKernelGGL
 // with a pair of library-owned events that take that dispatch's own start and
 // end timestamps: no marker packet goes between the kernels, so the timed
-// calls keep the untimed schedule.  One set of events per call, in a ring of
+// calls keep the untimed schedule, but for routing of at most kSmallTok tokens
+// (three kernels instead of one, each with a time of its own).  One set of events per call, in a ring of
 // `calls` sets; t_slot is the set of the call being enqueued (-1: untimed) and
 // t_role the kernel role about to be launched.
 // ---------------------------------------------------------------------------
@@ -174,9 +175,11 @@ int launch_gemm(GemmParams p, hipStream_t stream, int grid_override = 0) {
 }
 
 // MFMA shape of the 128x128-tile dense kernel (hkmoe_set_dense_mfma): 16 or 32.
-// 32x32x64 is the default: 2048^3 runs in 14.0 vs 15.1 us, 1024x4096x4096 in
-// 23.2 vs 24.7 us, 4096x2048x1024 in 16.8 vs 17.1 us (graph-replayed launches,
-// rotating operand copies, best of three interleaved rounds on one box).
+// 32x32x64 is the default from the time of four waves per workgroup, where it was
+// 4-7% faster.  On the eight waves of today the two are within 1-4%, 16x16x128 ahead
+// (bf16 output, rotating operand copies, graph-replayed launches, best of three
+// interleaved rounds on one box: 2048^3 13.3 / 13.7 us, 1024x4096x4096 21.6 / 22.2,
+// 4096x2048x1024 17.0 / 17.1).
 std::atomic<int> g_dense_mfma{32};
 
 // The dense GEMM on 128x128 tiles (gemm_small.hpp): one workgroup per tile,
@@ -1409,14 +1412,12 @@ int hkmoe_quant_tensor(const float* x, int64_t rows, int64_t cols, void* q, floa
   hipLaunchKernelGGL(fill_f32_kernel, dim3(1), dim3(1), 0, st, amax_ws, 0.0f);
   HK_TRY(check_launch("fill_f32_kernel"));
   const int grid = static_cast<int>(std::min<int64_t>((n + 1023) / 1024, 4096));
-  if (n > 0) {
-    // at most two workgroups per CU: each ends in one atomic on the same word,
-    // and they all end together (512 / 1024 / 2048 workgroups: 31 / 39 / 53 us for
-    // the three launches at 4096x4096)
-    const int agrid = static_cast<int>(std::min<int64_t>((n + 16383) / 16384, 512));
-    hipLaunchKernelGGL(amax_kernel, dim3(agrid), dim3(256), 0, st, x, n, amax_ws);
-    HK_TRY(check_launch("amax_kernel"));
-  }
+  // at most two workgroups per CU: each ends in one atomic on the same word,
+  // and they all end together (512 / 1024 / 2048 workgroups: 31 / 39 / 53 us for
+  // the three launches at 4096x4096)
+  const int agrid = static_cast<int>(std::min<int64_t>((n + 16383) / 16384, 512));
+  hipLaunchKernelGGL(amax_kernel, dim3(agrid), dim3(256), 0, st, x, n, amax_ws);
+  HK_TRY(check_launch("amax_kernel"));
   hipLaunchKernelGGL(quant_tensor_kernel, dim3(grid), dim3(256), 0, st, x, n, amax_ws,
                      static_cast<uint8_t*>(q), s);
   return check_launch("quant_tensor_kernel");

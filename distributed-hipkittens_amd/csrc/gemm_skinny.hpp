@@ -35,10 +35,8 @@ struct SkinnyParams {
 
 constexpr int kSkMaxLds = 160 * 1024;
 constexpr int sk_step_bytes(int mf, int nf, bool mx) { return (mf + nf) * 2048 + (mx ? 512 : 0); }
-// ring depth: what fits, at most 6 steps (one workgroup per CU)
-constexpr int sk_depth(int mf, int nf, int nw, bool mx) {
-  return kSkMaxLds / (sk_step_bytes(mf, nf, mx) * nw) < 6 ? kSkMaxLds / (sk_step_bytes(mf, nf, mx) * nw) : 6;
-}
+// ring depth: the steps that fit (one workgroup per CU), 2 to 5 for the strips in use
+constexpr int sk_depth(int mf, int nf, int nw, bool mx) { return kSkMaxLds / (sk_step_bytes(mf, nf, mx) * nw); }
 constexpr int sk_ring_bytes(int mf, int nf, int nw, bool mx) {
   return sk_depth(mf, nf, nw, mx) * nw * sk_step_bytes(mf, nf, mx);
 }

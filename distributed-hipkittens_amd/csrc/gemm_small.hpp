@@ -9,9 +9,10 @@
 // A K step is bounded by one wave's issue of fragment reads and DMA beside its
 // MFMAs: each wave overlaps its own LDS fragment reads of step kt+1 with its MFMAs
 // of step kt (two register sets of fragments), and the second wave of the SIMD fills
-// what is left (4 waves of 64x64, one per SIMD, read a quarter less from LDS but
-// took 13.28 us against 12.45 at 2048^3, 19.29 against 17.05 at 512x4096x4096, 30.6
-// against 26.8 at 1024x2048x7168).  A 4-deep LDS ring fed by buffer->LDS DMA keeps
+// what is left.  Against 4 waves of 64x64, one per SIMD, which read a quarter less
+// from LDS (graph-replayed launches, one box, operands resident / rotating over 512 MB):
+// 2048^3 12.7 -> 11.3 / 13.8 -> 13.7 us, 512x4096x4096 19.5 -> 16.8 / 21.4 -> 20.5,
+// 1024x2048x7168 30.6 -> 26.8 / 34.6 -> 33.1.  A 4-deep LDS ring fed by buffer->LDS DMA keeps
 // three K steps (96 KiB per CU) in flight (a fifth stage measured slower).  The
 // 2048^3 GEMM (config 1) is 256 such tiles, one per CU, where the 256x256 kernel has
 // 64.

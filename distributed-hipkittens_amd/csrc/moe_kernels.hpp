@@ -719,8 +719,8 @@ __device__ __forceinline__ float max_abs4(f32x4 v) {
 }
 
 // Four values / sc as e4m3 bytes.  Finite values take the division-free
-// quotient (quot_e4m3 with QuotScale; over 2.7e9 random and near-midpoint fp32
-// pairs with x <= 448 sc and x / sc >= 2^-10 it never differed from x / sc) and
+// quotient (quot_e4m3 with QuotScale: the theorem named there holds for every fp32 x
+// <= 448 sc with x / sc >= 2^-10, and below that both quotients round to 0) and
 // the packed conversion; a NaN or an infinite scale keeps the division and the
 // software conversion (NaN code 0x7f | sign).
 __device__ __forceinline__ uint32_t quant4(f32x4 v, float sc, const QuotScale& qs) {

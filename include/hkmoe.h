@@ -60,7 +60,9 @@ const char* hkmoe_last_error(void);
  * Dense FP8 GEMM  C[M,N] = (sa*sb) * sum_k A[m,k] * B[n,k]   (A . B^T, "TN")
  *   A [M,K] e4m3, B [N,K] e4m3, C [M,N] bf16 (RNE) or fp32.
  *   scale_a, scale_b: device fp32 scalars, or NULL for 1.0.
- *   Requires K % 128 == 0 and N % 256 == 0; M is arbitrary.
+ *   Requires K % 128 == 0 and N % 256 == 0; M is arbitrary.  fp32 accumulation;
+ *   the kernel, and with it the order of a row's sum over K, follows from M, N and
+ *   K, so a row's last bits may differ with the number of rows beside it.
  * Replaces the reference's dispatch_micro(A, B, C) (C = A . B^T, fp32 out):
  *   kernels/cdna3/gemm/fp8fp32/mi300x/8192_256_256_64_32/data_logs/
  *   0613_003858_outputs/256_256_64_32.cpp:202-212 and the FP8 GEMM kernels named
@@ -73,8 +75,8 @@ int hkmoe_gemm_fp8(const void* a, const void* b, void* c, int64_t m, int64_t n, 
 /*
  * MFMA shape of hkmoe_gemm_fp8's kernel for mid-sized problems (too few 256x256
  * tiles to fill the chip, e.g. 2048^3), which runs 128x128 tiles: 16 for
- * v_mfma_f32_16x16x128_f8f6f4, 32 for v_mfma_f32_32x32x64_f8f6f4 (the default:
- * 4-7% faster at 2048^3 and similar shapes).
+ * v_mfma_f32_16x16x128_f8f6f4, 32 for v_mfma_f32_32x32x64_f8f6f4 (the default;
+ * 1-4% apart).
  * Both give the same sums (fp32 accumulation in another order).  Replaces the
  * choice between the reference's mfma1616128 and mfma323264 wrappers
  * (include/cdna4/ops/warp/register/tile/mma.cuh:97-125).  Other values are
@@ -86,8 +88,8 @@ int hkmoe_get_dense_mfma(void);
 /*
  * Routing step 1: top-k + softmax weights + per-block expert histogram.
  *   logits [T,E] fp32 -> topk_idx [T,k] int32, topk_w [T,k] fp32.
- *   Order: descending logit, ties to the lower expert id.  Weights: softmax
- *   over the k selected logits.  block_counts: workspace [nblk, E] int32 with
+ *   Order: descending logit, ties to the lower expert id, a NaN below every
+ *   number.  Weights: softmax over the k selected logits.  block_counts: workspace [nblk, E] int32 with
  *   nblk = hkmoe_route_blocks(T).  E <= 1024, 1 <= k <= min(E, 32).
  * The reference has no router, histogram or permutation: the routing entry
  * points (this one, hkmoe_expert_offsets, hkmoe_scatter) and the MoE entry
@@ -299,8 +301,9 @@ size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t
  * 256*E, and not above), by an estimate of what they save (70 of 44 MB and 10 rows each
  * are enough), then on the auxiliary one at least 100.  Results are bit-identical
  * with the narrow path on or off.
- * cus == 0 turns it off; while 256x256 tiles exist the narrow kernels take at most three quarters of the device's CUs, whatever cus asks for (the
- * first wide GEMM keeps the rest); wide_share 1 or 2 runs the first wide GEMM on
+ * cus == 0 turns it off; while 256x256 tiles exist the narrow kernels take at most
+ * three quarters of the device's CUs, whatever cus asks for (the first wide GEMM
+ * keeps the rest); wide_share 1 or 2 runs the first wide GEMM on
  * (CUs - cus) workgroups while narrow experts exist; with 2 the narrow path's CUs
  * also join that GEMM's remaining tiles once both narrow GEMMs are done (a second
  * launch of it on the auxiliary stream), and the second wide GEMM waits for
@@ -371,8 +374,9 @@ int hkmoe_moe_forward(const void* x_q, const float* x_scale, const float* logits
  * per-tensor scales).  Every kernel runs on `stream`: the narrow path's auxiliary
  * stream is not used, so layers that hkmoe_moe_forward runs on one stream (see
  * hkmoe_set_narrow; every layer of the first two shapes above that fits the scratch)
- * take the same schedule here, and the rest run the 256x256 kernels alone.  The first call on a device looks up that device's scratch
- * address (hipGetSymbolAddress): make it outside graph capture.  All calls on
+ * take the same schedule here, and the rest run the 256x256 kernels alone.  The
+ * first call on a device looks up that device's scratch address
+ * (hipGetSymbolAddress): make it outside graph capture.  All calls on
  * one device share its scratch and each call leaves its intermediates there:
  * calls that overlap in time on one device (other streams, other threads)
  * race and must be serialised by the caller.
@@ -389,8 +393,8 @@ int hkmoe_moe_forward_noalloc(const void* x_q, const float* x_scale, const float
  *   hkmoe_quant_block:  q [B,R,C] e4m3, s [B, R/128, C/128] (128x128 blocks)
  *   hkmoe_quant_tensor: q [R,C], s [1]; amax_ws: one fp32 of device scratch.
  * Scale = amax/448 (1.0 for an all-zero block); q = e4m3(x / s) RNE, saturating.
- * Bit-exact for finite x; a NaN gives +-448 (0x7E | sign), and block maxima
- * skip NaNs.
+ * Bit-exact for finite x; a NaN gives the NaN code (0x7F | sign), and maxima skip
+ * NaNs.
  */
 int hkmoe_quant_group(const float* x, int64_t rows, int64_t cols, void* q, float* s,
                       hkmoe_stream_t stream);
@@ -431,7 +435,8 @@ int hkmoe_mx_pack_scales(const void* s, int64_t rows, int64_t cols, void* packed
  *     2^(sa[m,kb] - 127) * 2^(sb[n,kb] - 127) * sum_{k in kb} A[m,k] * B[n,k]
  *   A [M,K] e4m3 with packed scales a_scale [K/128, M64]; B [N,K] e4m3 with
  *   packed scales b_scale [K/128, N] (hkmoe_mx_pack_scales); fp32 accumulate,
- *   C bf16 (RNE) or fp32.  K % 128 == 0, N % 256 == 0, M arbitrary.
+ *   C bf16 (RNE) or fp32.  K % 128 == 0, N % 256 == 0, M arbitrary.  The order of a
+ *   row's sum follows from M, N and K, as in hkmoe_gemm_fp8.
  *   Replaces mxfp8_gemm_4wave_kernel (4_wave.cu:77-292), which is launched
  *   with the packed scales of prepare_mxfp8_data (4_wave.cu:377-448).
  */
