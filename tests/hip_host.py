@@ -53,7 +53,7 @@ def build_fake(directory):
 
 def run(fake_dir, snippet, timeout=60):
     """stdout lines of the snippet (it sees PRELUDE's names)."""
-    env = dict(os.environ, LD_LIBRARY_PATH=fake_dir)
+    env = dict(os.environ, LD_LIBRARY_PATH=":".join([fake_dir] + os.environ.get("LD_LIBRARY_PATH", "").split(":")).rstrip(":"))
     for name in ("HKMOE_NARROW_CUS", "HKMOE_NARROW_MAX", "HKMOE_NARROW_SHARE"):
         env.pop(name, None)
     res = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(snippet)], capture_output=True, text=True,
