@@ -299,8 +299,8 @@ size_t hkmoe_moe_workspace_size(int64_t num_tokens, int32_t num_experts, int32_t
  * least 256 experts where the routing leaves no expert above max_rows rows, or enough
  * narrow ones beside the larger: on one stream, up to T*top_k = 176*E (per-tensor:
  * 256*E, and not above), by an estimate of what they save (of 44 MB and 10 rows
- * each, 85 are enough, per-tensor 110), then on the auxiliary one at least 100.  Results are bit-identical
- * with the narrow path on or off.
+ * each, 85 are enough, per-tensor 110), then on the auxiliary one at least 100.
+ * Results are bit-identical with the narrow path on or off.
  * cus == 0 turns it off; while 256x256 tiles exist the narrow kernels take at most
  * three quarters of the device's CUs, whatever cus asks for (the first wide GEMM
  * keeps the rest); wide_share 1 or 2 runs the first wide GEMM on
